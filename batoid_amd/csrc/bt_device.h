@@ -22,9 +22,24 @@
 
 namespace bt {
 
+// Descriptors and coefficient tables are read through the constant address
+// space (no launch that reads them writes them, and every lane of a wave reads
+// one address: scalar loads), tables gathered per lane through the global
+// one.  The compiler infers this from generic pointers in small kernels only;
+// a plan kernel left with flat loads took twice the time.
+#define BT_CONSTANT __attribute__((address_space(4)))
+#define BT_GLOBAL __attribute__((address_space(1)))
+using SurfPtr = const BT_CONSTANT bt_surface*;
+using MediumPtr = const BT_CONSTANT bt_medium*;
+using ObscPtr = const BT_CONSTANT bt_obsc*;
+using StepPtr = const BT_CONSTANT bt_step*;
+using CoefPtr = const BT_CONSTANT double*;
+using TrimPtr = const BT_CONSTANT int*;
+using TablePtr = const BT_GLOBAL double*;
+
 // ---------------------------------------------------------------------------
-// sqrt(x) and 1/sqrt(x), correctly rounded, without range handling where it
-// cannot change a bit.
+// Square roots, reciprocal roots and quotients, correctly rounded, without
+// range handling where it cannot change a bit.
 //
 // The compiler's IEEE sqrt scales x < 2^-767 by 2^256 before the v_rsq_f64
 // estimate, refines it (g = x r, h = r/2; one coupled Goldschmidt step; two
@@ -32,27 +47,81 @@ namespace bt {
 // itself for +-0 and +inf.  Its IEEE division rescales operands of extreme
 // exponent (v_div_scale), refines v_rcp_f64 by two Newton steps, applies one
 // Markstein correction q + (n - d q) r, and patches special operands
-// (v_div_fixup).  For x in [2^-767, DBL_MAX] all of that range handling is
-// the identity: the scale factors are 2^0 and nothing is special, and the
-// root s lies in [2^-384, 2^512], where 1/s is not rescaled or patched
-// either (the quotient 1*r of the first step is r itself).  There the same
-// refinement steps run here without it; the range handling is 8 of the 18
-// vector instructions of a sqrt and 12 of the 29 of a 1/sqrt, the range
-// test that replaces it two compares.  Every other x (zero, tiny, negative,
-// infinite, NaN) takes the compiler's full sequence, so cr_sqrt(x) and
-// cr_rsqrt(x) are bit-identical to sqrt(x) and 1/sqrt(x) for every input
-// (bt_check_sqrt exposes both for testing).
+// (v_div_fixup).  Where no operand, quotient or remainder comes near the
+// ends of the exponent range all of that range handling is the identity, and
+// the *_plain functions below run the refinement alone.  They also share it:
+//  * the h that the root's iteration leaves is 1/(2 sqrt(x)) to ~2^-47, so
+//    one Newton step gives the reciprocal of a root (2 instructions instead
+//    of v_rcp_f64 and 4), and quotients by one denominator (x/r and y/r, the
+//    velocity by an index) share one reciprocal: a quotient is then 3
+//    instructions instead of 11 (v_rcp_f64 alone takes four issue slots);
+//  * a reciprocal y that is within an ulp of 1/d makes q = n y,
+//    q + (n - d q) y the correctly rounded quotient, which is the division's
+//    own last step, so the bits are the division's.
+// Every function of the trace exists in two forms.  The plain form (kPlain
+// true) runs these alone and notes in a Range what could have left their
+// range; a wave votes once on its lanes' Ranges, and only if one left it is
+// the work done again, by the whole wave, in the full form, whose roots and
+// divisions are the compiler's sequences.  The full form (the on-axis ray
+// r = 0, overflow) stays out of the plain form's registers.
+//
+// A Range is two running extremes in vector registers, an instruction or two
+// per value noted: the compares and scalar masks of a test at each root cost
+// the plan kernel of the analytic surfaces 11 % (1.93 against 1.73 ms for
+// 1e7 rays through twelve interfaces).  What is noted:
+//  * every argument of a root (a zero, a negative one, an overflow, a NaN);
+//  * the exponents of a ray's x and y at each surface and of its final
+//    velocity: nothing nonzero below 2^-601, so that no remainder n - d q of a
+//    quotient underflows.  (A difference of two doubles is 0 or at least an
+//    ulp of theirs, so tiny values come only from tiny values.)
+// One pair of operands is given up: n a power of two over a d whose
+// significand is all ones, where a reciprocal refined from a root's h rounds
+// the quotient down an ulp.
 // ---------------------------------------------------------------------------
+struct Range {
+    uint32_t high = 0;           // largest high word noted
+    int32_t low = 0;             // smallest exponent noted
+
+    // w > 0 expected: an overflow, a NaN or a negative w is out of range
+    __device__ __forceinline__ void above(double w)
+    {
+        high = max(high, (uint32_t)__double2hiint(w));
+    }
+    // as above, and zero too (the high word of a positive double below
+    // 2^-1022 is 0 only if it is below 2^-1042)
+    __device__ __forceinline__ void positive(double w)
+    {
+        high = max(high, (uint32_t)__double2hiint(w) - 1u);
+    }
+    __device__ __forceinline__ void positive(double w, double v)
+    {
+        high = max(max(high, (uint32_t)__double2hiint(w) - 1u),
+                   (uint32_t)__double2hiint(v) - 1u);
+    }
+    __device__ __forceinline__ void not_tiny(double a, double b)
+    {
+        low = min(min(low, __builtin_amdgcn_frexp_exp(a)), __builtin_amdgcn_frexp_exp(b));
+    }
+    __device__ __forceinline__ void leave() { high = ~0u; }
+    // below 2^601, and nothing nonzero below 2^-601
+    __device__ __forceinline__ bool plain() const
+    {
+        return (high < ((1023u + 601u) << 20)) & (low >= -600);
+    }
+};
+
+
 BT_DEV bool sqrt_in_plain_range(double x)
 {
     return x >= 0x1p-767 && x <= 0x1.fffffffffffffp+1023;
 }
 
-BT_DEV double sqrt_plain_range(double x)
+// sqrt(x); h becomes 1/(2 sqrt(x)) to ~2^-47.
+BT_DEV double sqrt_plain(double x, double& h)
 {
     const double r = __builtin_amdgcn_rsq(x);
     double g = x * r;
-    double h = r * 0.5;
+    h = r * 0.5;
     const double e = __builtin_fma(-h, g, 0.5);
     g = __builtin_fma(g, e, g);
     h = __builtin_fma(h, e, h);
@@ -62,27 +131,90 @@ BT_DEV double sqrt_plain_range(double x)
     return __builtin_fma(d, h, g);
 }
 
-BT_DEV double recip_plain_range(double s)
+// 1/d to within an ulp, from y0 = 1/d to ~2^-40 or better.
+BT_DEV double recip_refine(double d, double y0)
 {
-    double r = __builtin_amdgcn_rcp(s);
-    double e = __builtin_fma(-s, r, 1.0);
-    r = __builtin_fma(r, e, r);
-    e = __builtin_fma(-s, r, 1.0);
-    r = __builtin_fma(r, e, r);
-    const double rem = __builtin_fma(-s, r, 1.0);
-    return __builtin_fma(rem, r, r);
+    return __builtin_fma(y0, __builtin_fma(-d, y0, 1.0), y0);
+}
+
+// 1/g to within an ulp for g = sqrt_plain(x, h).
+BT_DEV double recip_root(double g, double h) { return recip_refine(g, h + h); }
+
+// 1/d to within an ulp.
+BT_DEV double recip_plain(double d)
+{
+    return recip_refine(d, recip_refine(d, __builtin_amdgcn_rcp(d)));
+}
+
+// n/d from y = 1/d to within an ulp.
+BT_DEV double div_plain(double n, double d, double y)
+{
+    const double q = n * y;
+    return __builtin_fma(__builtin_fma(-d, q, n), y, q);
+}
+
+// As div_plain, with the quotient's sign right for n = +-0 too.
+BT_DEV double div_plain_signed(double n, double d, double y)
+{
+    return __builtin_amdgcn_div_fixup(div_plain(n, d, y), d, n);
+}
+
+// 2^-200 <= |d| < 2^201, on the exponent bits (a scalar test where d is
+// wave-uniform).
+BT_DEV bool plain_exponent(double d)
+{
+    return (((uint32_t)__double2hiint(d) >> 20) & 0x7ffu) - (1023u - 200u) <= 400u;
+}
+
+// 1/sqrt(x), two roundings; g becomes sqrt(x).  (Not from h: next to 1 -- the
+// root of a unit velocity's square -- g is often 1 - 2^-53, whose reciprocal
+// rounds up from a hair above a midpoint, which the refinement of 2h misses.)
+BT_DEV double rsqrt_plain(double x, double& g)
+{
+    double h;
+    g = sqrt_plain(x, h);
+    const double y = recip_plain(g);
+    return __builtin_fma(__builtin_fma(-g, y, 1.0), y, y);
 }
 
 BT_DEV double cr_sqrt(double x)
 {
-    if (sqrt_in_plain_range(x)) return sqrt_plain_range(x);
+    double h;
+    if (__all(sqrt_in_plain_range(x))) return sqrt_plain(x, h);
     return __builtin_sqrt(x);
 }
 
 BT_DEV double cr_rsqrt(double x)                    // 1/sqrt(x): two roundings
 {
-    if (sqrt_in_plain_range(x)) return recip_plain_range(sqrt_plain_range(x));
+    double root;
+    if (__all(sqrt_in_plain_range(x))) return rsqrt_plain(x, root);
     return 1.0 / __builtin_sqrt(x);
+}
+
+// sqrt(x) and 1/sqrt(x) (two roundings) in either form; `root` becomes
+// sqrt(x), the reciprocal of the result to an ulp, or 0 in the full form.
+template <bool kPlain>
+BT_DEV double root_of(double x, Range& rg)
+{
+    if constexpr (kPlain) {
+        double h;
+        rg.positive(x);
+        return sqrt_plain(x, h);
+    } else {
+        return cr_sqrt(x);
+    }
+}
+
+template <bool kPlain>
+BT_DEV double recip_root_of(double x, double& root, Range& rg)
+{
+    if constexpr (kPlain) {
+        rg.positive(x);
+        return rsqrt_plain(x, root);
+    } else {
+        root = 0.0;
+        return cr_rsqrt(x);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -115,23 +247,23 @@ BT_DEV int cell_index(double u)
     return (int)f;
 }
 
-BT_DEV bool table_cell(const bt_surface* s, double x, double y, int& ix, int& iy)
+BT_DEV bool table_cell(SurfPtr s, double x, double y, int& ix, int& iy)
 {
     ix = cell_index((x - s->p[0])/s->p[2]);
     iy = cell_index((y - s->p[1])/s->p[3]);
     return !(ix >= s->n1-1 || ix < 0 || iy >= s->n2-1 || iy < 0);
 }
 
-BT_DEV double table_eval(const bt_surface* s, double x, double y)
+BT_DEV double table_eval(SurfPtr s, double x, double y)
 {
     int ix, iy;
     if (!table_cell(s, x, y, ix, iy))
         return s->flags ? __builtin_nan("") : 0.0;
     const double dx = s->p[2], dy = s->p[3];
-    const double* __restrict__ z = s->a0;
-    const double* __restrict__ zx = s->a1;
-    const double* __restrict__ zy = s->a2;
-    const double* __restrict__ zxy = s->a3;
+    const TablePtr z = (TablePtr)s->a0;
+    const TablePtr zx = (TablePtr)s->a1;
+    const TablePtr zy = (TablePtr)s->a2;
+    const TablePtr zxy = (TablePtr)s->a3;
     double xgrid = s->p[0] + ix*dx;
     double ygrid = s->p[1] + iy*dy;
     double xfrac = (x - xgrid)/dx;
@@ -144,7 +276,7 @@ BT_DEV double table_eval(const bt_surface* s, double x, double y)
     return spline1(yfrac, val0, val1, der0*dy, der1*dy);
 }
 
-BT_DEV void table_grad(const bt_surface* s, double x, double y,
+BT_DEV void table_grad(SurfPtr s, double x, double y,
                        double& dzdx, double& dzdy)
 {
     int ix, iy;
@@ -154,10 +286,10 @@ BT_DEV void table_grad(const bt_surface* s, double x, double y,
         return;
     }
     const double dx = s->p[2], dy = s->p[3];
-    const double* __restrict__ z = s->a0;
-    const double* __restrict__ zx = s->a1;
-    const double* __restrict__ zy = s->a2;
-    const double* __restrict__ zxy = s->a3;
+    const TablePtr z = (TablePtr)s->a0;
+    const TablePtr zx = (TablePtr)s->a1;
+    const TablePtr zy = (TablePtr)s->a2;
+    const TablePtr zxy = (TablePtr)s->a3;
     double xgrid = s->p[0] + ix*dx;
     double ygrid = s->p[1] + iy*dy;
     double xfrac = (x - xgrid)/dx;
@@ -185,12 +317,12 @@ BT_DEV void table_grad(const bt_surface* s, double x, double y,
 // ---------------------------------------------------------------------------
 // 2-D Horner (src/polynomialSurface.cpp:50-66)
 // ---------------------------------------------------------------------------
-BT_DEV double horner2d(double x, double y, const double* __restrict__ c,
+BT_DEV double horner2d(double x, double y, CoefPtr c,
                        int nx, int ny)
 {
     double r = 0.0;
     for (int i = ny-1; i >= 0; i--) {
-        const double* row = c + (int64_t)i*nx;
+        const CoefPtr row = c + (int64_t)i*nx;
         double h = 0.0;
         for (int j = nx-1; j >= 0; j--) { h *= y; h += row[j]; }
         r *= x;
@@ -207,14 +339,14 @@ BT_DEV double horner2d(double x, double y, const double* __restrict__ c,
 // 0.0 therefore gives the same bits, and rows of only +0.0 add exactly +0.0
 // where the full loop does.  A wave with any non-finite argument (0*inf is
 // NaN inside the skipped steps) runs the full loop.
-BT_DEV double horner2d_trim(double x, double y, const double* __restrict__ c,
-                            int nx, int ny, const int* __restrict__ trim)
+BT_DEV double horner2d_trim(double x, double y, CoefPtr c,
+                            int nx, int ny, TrimPtr trim)
 {
     if (!trim || !__all(__builtin_isfinite(x) && __builtin_isfinite(y)))
         return horner2d(x, y, c, nx, ny);
     double r = 0.0;
     for (int i = trim[0]; i >= 0; i--) {
-        const double* row = c + (int64_t)i*nx;
+        const CoefPtr row = c + (int64_t)i*nx;
         double h = 0.0;
         for (int j = trim[1 + i] - 1; j >= 0; j--) { h *= y; h += row[j]; }
         r *= x;
@@ -225,167 +357,243 @@ BT_DEV double horner2d_trim(double x, double y, const double* __restrict__ c,
 
 // Trim tables of a POLYNOMIAL record's coefficient, x-gradient and
 // y-gradient tables, in that order, in the record's optional int32 table a3.
-BT_DEV const int* poly_trim(const bt_surface* s, int which)
+BT_DEV TrimPtr poly_trim(SurfPtr s, int which)
 {
-    const int* t = reinterpret_cast<const int*>(s->a3);
-    if (!t) return nullptr;
+    if (!s->a3) return nullptr;
+    const TrimPtr t = (TrimPtr)reinterpret_cast<const int*>(s->a3);
     if (which == 0) return t;
     return t + (1 + s->n2) + (which - 1) * s->n2;
 }
 
-// table_eval and table_grad at one point, sharing the cell and its 16 table
-// values; each result is bit-identical to the separate function's.
-BT_DEV void table_eval_grad(const bt_surface* s, double x, double y, double& val,
-                            double& dzdx, double& dzdy)
+// Table `which` (0: coefficients, 1, 2: x and y gradients) of a POLYNOMIAL
+// record at (u, v) from its origin.
+BT_DEV double poly_table(SurfPtr s, int which, double u, double v)
 {
-    int ix, iy;
-    if (!table_cell(s, x, y, ix, iy)) {
-        double v = s->flags ? __builtin_nan("") : 0.0;
-        val = v; dzdx = v; dzdy = v;
-        return;
+    const CoefPtr c = (CoefPtr)(which == 0 ? s->a0 : which == 1 ? s->a1 : s->a2);
+    const int nx = s->n1 - (which > 0), ny = s->n2 - (which > 0);
+    const TrimPtr trim = poly_trim(s, which);
+    return horner2d_trim(u, v, c, nx, ny, trim);
+}
+
+// Sag and / or normal of a Bicubic at one point (bicubic.cpp:19-40), sharing
+// the cell and its 16 table values; each result is bit-identical to
+// table_eval's and table_grad's.  `inv`: 1/nz to an ulp, or 0.  With the
+// record's optional reciprocals of the grid steps the four (sag) or six
+// (normal) divisions by dx and dy, ten at a point of a Newton iteration, are
+// three or four instructions each.
+template <bool kPlain, bool kSag, bool kNormal>
+BT_DEV void table_point(SurfPtr s, double x, double y, double& sag, double& nx,
+                        double& ny, double& nz, double& inv, Range& rg)
+{
+    if constexpr (!kPlain) {
+        if constexpr (kSag) sag = table_eval(s, x, y);
+        if constexpr (kNormal) {
+            double dzdx, dzdy;
+            table_grad(s, x, y, dzdx, dzdy);
+            inv = 0.0;
+            if (__builtin_isnan(dzdx)) {
+                nx = __builtin_nan(""); ny = nx; nz = nx;
+            } else {
+                nz = cr_rsqrt(1 + dzdx*dzdx + dzdy*dzdy);
+                nx = -dzdx*nz;
+                ny = -dzdy*nz;
+            }
+        }
+    } else {
+        if (s->n1 < 2 || s->n2 < 2) {                // no cell to read
+            rg.leave();
+            if constexpr (kSag) sag = 0.0;
+            if constexpr (kNormal) { nx = 0.0; ny = 0.0; nz = 1.0; inv = 1.0; }
+            return;
+        }
+        const double dx = s->p[2], dy = s->p[3], rx = s->p[4], ry = s->p[5];
+        const double x0 = s->p[0], y0 = s->p[1];
+        // not the correctly rounded 1/dx and 1/dy (0: not given)
+        if (!plain_exponent(dx) || !plain_exponent(dy)
+            || !(fabs(__builtin_fma(-dx, rx, 1.0)) <= 0x1p-53)
+            || !(fabs(__builtin_fma(-dy, ry, 1.0)) <= 0x1p-53))
+            rg.leave();
+        const double ux = x - x0, uy = y - y0;
+        const double fx = floor(div_plain(ux, dx, rx)), fy = floor(div_plain(uy, dy, ry));
+        const bool inside = (fx >= 0.0) & (fx < (double)(s->n1 - 1)) & (fy >= 0.0)
+                            & (fy < (double)(s->n2 - 1));
+        const TablePtr z = (TablePtr)s->a0;
+        const TablePtr zx = (TablePtr)s->a1;
+        const TablePtr zy = (TablePtr)s->a2;
+        const TablePtr zxy = (TablePtr)s->a3;
+        // a lane outside the table reads its first cell
+        const int64_t k0 = inside ? (int64_t)s->n1*(int)fy + (int)fx : 0, k1 = k0 + s->n1;
+        const double z00 = z[k0], z01 = z[k0+1], z10 = z[k1], z11 = z[k1+1];
+        const double x00 = zx[k0], x01 = zx[k0+1], x10 = zx[k1], x11 = zx[k1+1];
+        const double y00 = zy[k0], y01 = zy[k0+1], y10 = zy[k1], y11 = zy[k1+1];
+        const double c00 = zxy[k0], c01 = zxy[k0+1], c10 = zxy[k1], c11 = zxy[k1+1];
+        const double xn = x - (x0 + fx*dx), yn = y - (y0 + fy*dy);
+        const double xfrac = div_plain_signed(xn, dx, rx);
+        const double yfrac = div_plain_signed(yn, dy, ry);
+        double ts = 0.0, dzdx = 0.0, dzdy = 0.0;
+        if constexpr (kSag) {
+            double val0 = spline1(xfrac, z00, z01, x00*dx, x01*dx);
+            double val1 = spline1(xfrac, z10, z11, x10*dx, x11*dx);
+            double der0 = spline1(xfrac, y00, y01, c00*dx, c01*dx);
+            double der1 = spline1(xfrac, y10, y11, c10*dx, c11*dx);
+            ts = spline1(yfrac, val0, val1, der0*dy, der1*dy);
+        }
+        if constexpr (kNormal) {
+            double val0 = grad1(xfrac, z00, z01, x00*dx, x01*dx);
+            double val1 = grad1(xfrac, z10, z11, x10*dx, x11*dx);
+            double der0 = grad1(xfrac, y00, y01, c00*dx, c01*dx);
+            double der1 = grad1(xfrac, y10, y11, c10*dx, c11*dx);
+            const double gx = spline1(yfrac, val0, val1, der0*dy, der1*dy);
+            val0 = grad1(yfrac, z00, z10, y00*dy, y10*dy);
+            val1 = grad1(yfrac, z01, z11, y01*dy, y11*dy);
+            der0 = grad1(yfrac, x00, x10, c00*dy, c10*dy);
+            der1 = grad1(yfrac, x01, x11, c01*dy, c11*dy);
+            const double gy = spline1(xfrac, val0, val1, der0*dx, der1*dx);
+            dzdx = div_plain_signed(gx, dx, rx);
+            dzdy = div_plain_signed(gy, dy, ry);
+            rg.not_tiny(gx, gy);
+        }
+        if (!__all(inside)) {                        // outside: NaN or 0 (table.cpp:60-66)
+            const double v = s->flags ? __builtin_nan("") : 0.0;
+            ts = inside ? ts : v;
+            dzdx = inside ? dzdx : v;
+            dzdy = inside ? dzdy : v;
+        }
+        if constexpr (kSag) sag = ts;
+        if constexpr (kNormal) {
+            const double w = 1 + dzdx*dzdx + dzdy*dzdy;
+            rg.above(__builtin_fmax(w, 1.0));        // NaN slopes (outside): a NaN normal
+            nz = rsqrt_plain(w, inv);
+            nx = -dzdx*nz;
+            ny = -dzdy*nz;
+        }
     }
-    const double dx = s->p[2], dy = s->p[3];
-    const double* __restrict__ z = s->a0;
-    const double* __restrict__ zx = s->a1;
-    const double* __restrict__ zy = s->a2;
-    const double* __restrict__ zxy = s->a3;
-    double xgrid = s->p[0] + ix*dx;
-    double ygrid = s->p[1] + iy*dy;
-    double xfrac = (x - xgrid)/dx;
-    double yfrac = (y - ygrid)/dy;
-    const int64_t k0 = (int64_t)s->n1*iy + ix, k1 = k0 + s->n1;
-    const double z00 = z[k0], z01 = z[k0+1], z10 = z[k1], z11 = z[k1+1];
-    const double x00 = zx[k0], x01 = zx[k0+1], x10 = zx[k1], x11 = zx[k1+1];
-    const double y00 = zy[k0], y01 = zy[k0+1], y10 = zy[k1], y11 = zy[k1+1];
-    const double c00 = zxy[k0], c01 = zxy[k0+1], c10 = zxy[k1], c11 = zxy[k1+1];
-
-    double val0 = spline1(xfrac, z00, z01, x00*dx, x01*dx);
-    double val1 = spline1(xfrac, z10, z11, x10*dx, x11*dx);
-    double der0 = spline1(xfrac, y00, y01, c00*dx, c01*dx);
-    double der1 = spline1(xfrac, y10, y11, c10*dx, c11*dx);
-    val = spline1(yfrac, val0, val1, der0*dy, der1*dy);
-
-    val0 = grad1(xfrac, z00, z01, x00*dx, x01*dx);
-    val1 = grad1(xfrac, z10, z11, x10*dx, x11*dx);
-    der0 = grad1(xfrac, y00, y01, c00*dx, c01*dx);
-    der1 = grad1(xfrac, y10, y11, c10*dx, c11*dx);
-    dzdx = spline1(yfrac, val0, val1, der0*dy, der1*dy)/dx;
-
-    val0 = grad1(yfrac, z00, z10, y00*dy, y10*dy);
-    val1 = grad1(yfrac, z01, z11, y01*dy, y11*dy);
-    der0 = grad1(yfrac, x00, x10, c00*dy, c10*dy);
-    der1 = grad1(yfrac, x01, x11, c01*dy, c11*dy);
-    dzdy = spline1(xfrac, val0, val1, der0*dx, der1*dx)/dy;
 }
 
 // ---------------------------------------------------------------------------
 // Quadric family (src/quadric.cpp, src/asphere.cpp)
 // ---------------------------------------------------------------------------
-BT_DEV double quadric_sag(const bt_surface* s, double x, double y)
+// result + sum of an Asphere's n even terms c[i] r2^(i+1) (asphere.cpp:37-46),
+// or its slope's dc[i] r r2^i (asphere.cpp:53-59): term starts at the first
+// power and grows by r2.  (All coefficients in one 64-byte scalar load
+// instead of a load per term: the same time on the analytic kernel, 4 % more
+// on the Sum kernels, whose scalar registers are short.)
+BT_DEV double even_terms(CoefPtr c, int n, double result, double term, double r2)
 {
-    const double R = s->p[0];
-    double r2 = x*x + y*y;
-    if (R != 0)
-        return r2/(R*(1.+cr_sqrt(1.-r2*s->p[8])));
-    return 0.0;
-}
-
-BT_DEV double quadric_dzdr(const bt_surface* s, double r)
-{
-    const double R = s->p[0];
-    if (R != 0.0)
-        return r/(R*cr_sqrt(1-r*r*s->p[8]));
-    return 0.0;
-}
-
-BT_DEV double asphere_dzdr(const bt_surface* s, double r)
-{
-    double result = quadric_dzdr(s, r);
-    double rr = r*r;
-    double rrr = r;
-    const double* __restrict__ dc = s->a1;
-    const int n = s->n1;
     for (int i = 0; i < n; i++) {
-        result += dc[i]*rrr;
-        rrr *= rr;
+        result += c[i]*term;
+        term *= r2;
     }
     return result;
 }
 
-BT_DEV double asphere_sag(const bt_surface* s, double x, double y)
-{                                                    // asphere.cpp:37-46
-    double r2 = x*x + y*y;
-    double rr = 1.0;
-    double result = quadric_sag(s, x, y);
-    const double* __restrict__ c = s->a0;
-    const int n = s->n1;
-    for (int i = 0; i < n; i++) {
-        rr *= r2;
-        result += c[i]*rr;
-    }
-    return result;
-}
-
-// Normal of a Quadric (kAsphere false) or an Asphere (true): quadric.cpp:27-39,
-// asphere.cpp:48-62.
-template <bool kAsphere>
-BT_DEV void conic_normal(const bt_surface* s, double x, double y,
-                         double& nx, double& ny, double& nz)
+// Sag and / or normal of a Quadric (kAsphere false) or an Asphere (true) at
+// one point: quadric.cpp:18-39, asphere.cpp:37-62.  `inv`: 1/nz to an ulp,
+// or 0.  Bound by FP64 issue: the normal's three divisions and the reciprocal
+// of its third root come from the roots' own h here.
+template <bool kPlain, bool kAsphere, bool kSag, bool kNormal>
+BT_DEV void conic_point(SurfPtr s, double x, double y, double& sag, double& nx,
+                        double& ny, double& nz, double& inv, Range& rg)
 {
-    double r = cr_sqrt(x*x + y*y);
-    if (r == 0.0) {
-        nx = 0.0; ny = 0.0; nz = 1.0;
+    const double R = s->p[0], cp1R2 = s->p[8];
+    const double r2 = x*x + y*y;
+    if constexpr (kPlain) {
+        if (!plain_exponent(R)) rg.leave();
+        if constexpr (kSag) {
+            const double v = 1.-r2*cp1R2;
+            rg.positive(v);
+            double h;
+            const double d = R*(1.+sqrt_plain(v, h));
+            sag = div_plain(r2, d, recip_plain(d));
+            if constexpr (kAsphere) sag = even_terms((CoefPtr)s->a0, s->n1, sag, r2, r2);
+        }
+        if constexpr (kNormal) {
+            double hr, hu;
+            const double r = sqrt_plain(r2, hr);
+            const double u = 1-r*r*cp1R2;
+            const double d = R*sqrt_plain(u, hu);
+            const double y0 = (hu + hu) * (R*s->p[3]);   // 1/sqrt(u) * (R * 1/R/R)
+            double dzdr = div_plain(r, d, recip_refine(d, y0));
+            if constexpr (kAsphere) dzdr = even_terms((CoefPtr)s->a1, s->n1, dzdr, r, r*r);
+            const double w = 1+dzdr*dzdr;
+            rg.above(w);                                 // a NaN for r2 = 0 or u = 0
+            nz = rsqrt_plain(w, inv);
+            const double yr = recip_root(r, hr);
+            nx = -div_plain_signed(x, r, yr)*dzdr*nz;
+            ny = -div_plain_signed(y, r, yr)*dzdr*nz;
+        }
     } else {
-        double dzdr = kAsphere ? asphere_dzdr(s, r) : quadric_dzdr(s, r);
-        nz = cr_rsqrt(1+dzdr*dzdr);
-        nx = -x/r*dzdr*nz;
-        ny = -y/r*dzdr*nz;
+        if constexpr (kSag) {
+            sag = R != 0 ? r2/(R*(1.+cr_sqrt(1.-r2*cp1R2))) : 0.0;
+            if constexpr (kAsphere) sag = even_terms((CoefPtr)s->a0, s->n1, sag, r2, r2);
+        }
+        if constexpr (kNormal) {
+            const double r = cr_sqrt(r2);
+            inv = 0.0;
+            if (r == 0.0) {
+                nx = 0.0; ny = 0.0; nz = 1.0;
+            } else {
+                double dzdr = R != 0.0 ? r/(R*cr_sqrt(1-r*r*cp1R2)) : 0.0;
+                if constexpr (kAsphere)
+                    dzdr = even_terms((CoefPtr)s->a1, s->n1, dzdr, r, r*r);
+                nz = cr_rsqrt(1+dzdr*dzdr);
+                nx = -x/r*dzdr*nz;
+                ny = -y/r*dzdr*nz;
+            }
+        }
     }
 }
 
-BT_DEV double poly_sag(const bt_surface* s, double x, double y)
-{                                                    // polynomialSurface.cpp:35-37
-    return horner2d_trim(x-s->p[0], y-s->p[1], s->a0, s->n1, s->n2, poly_trim(s, 0));
+// Normal of a Sphere (sphere.cpp:23-35, 66-69).
+template <bool kPlain>
+BT_DEV void sphere_normal(SurfPtr s, double x, double y, double& nx, double& ny,
+                          double& nz, double& inv, Range& rg)
+{
+    const double Rinv = s->p[2];
+    const double rsqr = x*x + y*y;
+    if constexpr (kPlain) {
+        double hr, hu;
+        const double r = sqrt_plain(rsqr, hr);
+        const double rat = r*Rinv;
+        const double u = 1-rat*rat;
+        const double su = sqrt_plain(u, hu);
+        const double dzdr = div_plain(rat, su, recip_root(su, hu));
+        const double w = 1+dzdr*dzdr;
+        if (!plain_exponent(Rinv)) rg.leave();
+        rg.above(w);                                     // a NaN for rsqr = 0 or u = 0
+        nz = rsqrt_plain(w, inv);
+        const double yr = recip_root(r, hr);
+        nx = -div_plain_signed(x, r, yr)*dzdr*nz;
+        ny = -div_plain_signed(y, r, yr)*dzdr*nz;
+    } else {
+        inv = 0.0;
+        if (s->p[0] == 0.0 || rsqr == 0.0) {
+            nx = 0.0; ny = 0.0; nz = 1.0;
+        } else {
+            const double r = cr_sqrt(rsqr);
+            const double rat = r*Rinv;
+            const double dzdr = rat/cr_sqrt(1-rat*rat);
+            nz = cr_rsqrt(1+dzdr*dzdr);
+            nx = -x/r*dzdr*nz;
+            ny = -y/r*dzdr*nz;
+        }
+    }
 }
 
-BT_DEV void poly_normal(const bt_surface* s, double x, double y,
-                        double& nx, double& ny, double& nz)
+BT_DEV double poly_sag(SurfPtr s, double x, double y)
+{                                                    // polynomialSurface.cpp:35-37
+    return poly_table(s, 0, x-s->p[0], y-s->p[1]);
+}
+
+template <bool kPlain>
+BT_DEV void poly_normal(SurfPtr s, double x, double y, double& nx, double& ny,
+                        double& nz, double& inv, Range& rg)
 {                                                    // polynomialSurface.cpp:39-48
-    double gx = -horner2d_trim(x-s->p[0], y-s->p[1], s->a1, s->n1-1, s->n2-1, poly_trim(s, 1));
-    double gy = -horner2d_trim(x-s->p[0], y-s->p[1], s->a2, s->n1-1, s->n2-1, poly_trim(s, 2));
-    nz = cr_rsqrt(gx*gx + gy*gy + 1);
+    double gx = -poly_table(s, 1, x-s->p[0], y-s->p[1]);
+    double gy = -poly_table(s, 2, x-s->p[0], y-s->p[1]);
+    nz = recip_root_of<kPlain>(gx*gx + gy*gy + 1, inv, rg);
     nx = gx*nz;
     ny = gy*nz;
-}
-
-BT_DEV void table_normal(const bt_surface* s, double x, double y,
-                         double& nx, double& ny, double& nz)
-{                                                    // bicubic.cpp:23-40
-    double dxdz, dydz;
-    table_grad(s, x, y, dxdz, dydz);
-    if (__builtin_isnan(dxdz)) {
-        nx = __builtin_nan(""); ny = nx; nz = nx;
-        return;
-    }
-    nz = cr_rsqrt(1 + dxdz*dxdz + dydz*dydz);
-    nx = -dxdz*nz;
-    ny = -dydz*nz;
-}
-
-// Bicubic sag and normal at one point, sharing the cell (bit-identical to
-// table_eval and table_normal).
-BT_DEV void table_sag_normal(const bt_surface* s, double x, double y, double& sag,
-                             double& nx, double& ny, double& nz)
-{                                                    // bicubic.cpp:19-40
-    double dxdz, dydz;
-    table_eval_grad(s, x, y, sag, dxdz, dydz);
-    if (__builtin_isnan(dxdz)) {
-        nx = __builtin_nan(""); ny = nx; nz = nx;
-        return;
-    }
-    nz = cr_rsqrt(1 + dxdz*dxdz + dydz*dydz);
-    nx = -dxdz*nz;
-    ny = -dydz*nz;
 }
 
 // ---------------------------------------------------------------------------
@@ -412,6 +620,12 @@ constexpr int kKindsAnalytic = 1;
 constexpr int kKindsSumAPB = 2;
 constexpr int kKindsFlatSums = 3;
 
+// Kind sets whose interactions run plain first.  kKindsAll, whose nested Sums
+// are inlined to three levels, keeps the full form alone: two forms of it
+// would double the largest kernels for the rarest optics.
+template <int K>
+constexpr bool kVoted = K != kKindsAll;
+
 // The kind set of leaves (records that are not Sums) under set K.
 constexpr int leaf_set(int K)
 {
@@ -419,24 +633,26 @@ constexpr int leaf_set(int K)
 }
 
 // A Sum record laid out as kKindsSumAPB requires (records s+1..s+3 follow it).
-BT_DEV bool sum_is_apb(const bt_surface* s)
+BT_DEV bool sum_is_apb(SurfPtr s)
 {
     return s->nchild == 3 && s[1].kind == BT_ASPHERE && s[2].kind == BT_POLYNOMIAL &&
            s[3].kind == BT_BICUBIC;
 }
 
 // ---------------------------------------------------------------------------
-// Leaf surfaces: sag and normal
+// Leaf surfaces: sag and normal.  `inv` beside a normal is 1/nz to an ulp in
+// the plain form: a Sum's slopes nx/nz and ny/nz start from it.
 // ---------------------------------------------------------------------------
-template <int K = kKindsAll>
-BT_DEV double leaf_sag(const bt_surface* s, double x, double y)
+template <int K, bool kPlain>
+BT_DEV double leaf_sag(SurfPtr s, double x, double y, Range& rg)
 {
+    double sag, nx, ny, nz, inv;
     switch (s->kind) {
     case BT_PLANE:                                   // plane.cpp:15-17
         return 0.0;
     case BT_SPHERE:                                  // sphere.cpp:17-21
         if (s->p[0] != 0)
-            return s->p[0]*(1-cr_sqrt(1-(x*x + y*y)*s->p[3]));
+            return s->p[0]*(1-root_of<kPlain>(1-(x*x + y*y)*s->p[3], rg));
         return 0.0;
     case BT_PARABOLOID:                              // paraboloid.cpp:17-23
         if (s->p[0] != 0) {
@@ -445,13 +661,18 @@ BT_DEV double leaf_sag(const bt_surface* s, double x, double y)
         }
         return 0.0;
     case BT_QUADRIC:                                 // quadric.cpp:18-25
-        return quadric_sag(s, x, y);
+        conic_point<kPlain, false, true, false>(s, x, y, sag, nx, ny, nz, inv, rg);
+        return sag;
     case BT_ASPHERE:                                 // asphere.cpp:37-46
-        return asphere_sag(s, x, y);
+        conic_point<kPlain, true, true, false>(s, x, y, sag, nx, ny, nz, inv, rg);
+        return sag;
     case BT_TILTED:                                  // tilted.cpp:16-18
         return x*s->p[0] + y*s->p[1];
     case BT_BICUBIC:                                 // bicubic.cpp:19-21
-        if constexpr (K == kKindsAll) return table_eval(s, x, y);
+        if constexpr (K == kKindsAll) {
+            table_point<kPlain, true, false>(s, x, y, sag, nx, ny, nz, inv, rg);
+            return sag;
+        }
         break;
     case BT_POLYNOMIAL:                              // polynomialSurface.cpp:35-37
         if constexpr (K == kKindsAll) return poly_sag(s, x, y);
@@ -460,93 +681,105 @@ BT_DEV double leaf_sag(const bt_surface* s, double x, double y)
     return __builtin_nan("");
 }
 
-template <int K = kKindsAll>
-BT_DEV void leaf_normal(const bt_surface* s, double x, double y,
-                        double& nx, double& ny, double& nz)
+template <int K, bool kPlain>
+BT_DEV void leaf_normal(SurfPtr s, double x, double y,
+                        double& nx, double& ny, double& nz, double& inv, Range& rg)
 {
+    double sag;
+    inv = 0.0;
     switch (s->kind) {
     case BT_PLANE:                                   // plane.cpp:19-23
-        nx = 0.0; ny = 0.0; nz = 1.0;
+        nx = 0.0; ny = 0.0; nz = 1.0; inv = 1.0;
         return;
-    case BT_SPHERE: {                                // sphere.cpp:23-35, 66-69
-        double rsqr = x*x + y*y;
-        if (s->p[0] == 0.0 || rsqr == 0.0) {
-            nx = 0.0; ny = 0.0; nz = 1.0;
-        } else {
-            double r = cr_sqrt(rsqr);
-            double rat = r*s->p[2];
-            double dzdr = rat/cr_sqrt(1-rat*rat);
-            nz = cr_rsqrt(1+dzdr*dzdr);
-            nx = -x/r*dzdr*nz;
-            ny = -y/r*dzdr*nz;
-        }
+    case BT_SPHERE:                                  // sphere.cpp:23-35, 66-69
+        sphere_normal<kPlain>(s, x, y, nx, ny, nz, inv, rg);
         return;
-    }
     case BT_PARABOLOID: {                            // paraboloid.cpp:25-37
         if (s->p[0] == 0) {
-            nx = 0.0; ny = 0.0; nz = 1.0;
+            nx = 0.0; ny = 0.0; nz = 1.0; inv = 1.0;
         } else {
             const double Rinv = s->p[1];
-            nz = cr_rsqrt(1+(x*x+y*y)*Rinv*Rinv);
+            nz = recip_root_of<kPlain>(1+(x*x+y*y)*Rinv*Rinv, inv, rg);
             nx = -x*Rinv*nz;
             ny = -y*Rinv*nz;
         }
         return;
     }
     case BT_QUADRIC:                                 // quadric.cpp:27-39
-    case BT_ASPHERE: {                               // asphere.cpp:48-62
-        double r = cr_sqrt(x*x + y*y);
-        if (r == 0.0) {
-            nx = 0.0; ny = 0.0; nz = 1.0;
-        } else {
-            double dzdr = (s->kind == BT_QUADRIC) ? quadric_dzdr(s, r)
-                                                  : asphere_dzdr(s, r);
-            nz = cr_rsqrt(1+dzdr*dzdr);
-            nx = -x/r*dzdr*nz;
-            ny = -y/r*dzdr*nz;
-        }
+        conic_point<kPlain, false, false, true>(s, x, y, sag, nx, ny, nz, inv, rg);
         return;
-    }
+    case BT_ASPHERE:                                 // asphere.cpp:48-62
+        conic_point<kPlain, true, false, true>(s, x, y, sag, nx, ny, nz, inv, rg);
+        return;
     case BT_TILTED: {                                // tilted.cpp:20-27
         const double tx = s->p[0], ty = s->p[1];
         nx = -tx;
         ny = -ty;
-        nz = cr_sqrt(1 - tx*tx - ty*ty);
+        nz = root_of<kPlain>(1 - tx*tx - ty*ty, rg);
+        if constexpr (kPlain) inv = recip_plain(nz);
         return;
     }
     case BT_BICUBIC:                                 // bicubic.cpp:23-40
-        if constexpr (K == kKindsAll) { table_normal(s, x, y, nx, ny, nz); return; }
+        if constexpr (K == kKindsAll) {
+            table_point<kPlain, false, true>(s, x, y, sag, nx, ny, nz, inv, rg);
+            return;
+        }
         break;
     case BT_POLYNOMIAL:                              // polynomialSurface.cpp:39-48
-        if constexpr (K == kKindsAll) { poly_normal(s, x, y, nx, ny, nz); return; }
+        if constexpr (K == kKindsAll) { poly_normal<kPlain>(s, x, y, nx, ny, nz, inv, rg); return; }
         break;
     }
     nx = __builtin_nan(""); ny = nx; nz = nx;
 }
 
-// Sag and normal at one point (the reference evaluates them separately; the
-// results here are bit-identical, with shared work evaluated once).
-template <int K = kKindsAll>
-BT_DEV void leaf_sag_normal(const bt_surface* s, double x, double y, double& sag,
-                            double& nx, double& ny, double& nz)
+// Sag and / or normal at one point (the reference evaluates them separately;
+// the results here are bit-identical, with shared work evaluated once).
+template <int K, bool kPlain, bool kSag, bool kNormal>
+BT_DEV void leaf_point(SurfPtr s, double x, double y, double& sag,
+                       double& nx, double& ny, double& nz, double& inv, Range& rg)
 {
-    if (K == kKindsAll && s->kind == BT_BICUBIC) {
-        table_sag_normal(s, x, y, sag, nx, ny, nz);
-        return;
+    if constexpr (kSag && kNormal) {
+        if (s->kind == BT_ASPHERE) {
+            conic_point<kPlain, true, true, true>(s, x, y, sag, nx, ny, nz, inv, rg);
+            return;
+        }
+        if constexpr (K == kKindsAll) {
+            if (s->kind == BT_BICUBIC) {
+                table_point<kPlain, true, true>(s, x, y, sag, nx, ny, nz, inv, rg);
+                return;
+            }
+        }
     }
-    sag = leaf_sag<K>(s, x, y);
-    leaf_normal<K>(s, x, y, nx, ny, nz);
+    if constexpr (kSag) sag = leaf_sag<K, kPlain>(s, x, y, rg);
+    if constexpr (kNormal) leaf_normal<K, kPlain>(s, x, y, nx, ny, nz, inv, rg);
 }
 
-BT_DEV void add_slope(double& sx, double& sy, double nx, double ny, double nz)
+// sx += nx/nz, sy += ny/nz; plain: from inv = 1/nz to an ulp.
+template <bool kPlain>
+BT_DEV void add_slope(double& sx, double& sy, double nx, double ny, double nz, double inv)
 {
-    sx += nx/nz;
-    sy += ny/nz;
+    if constexpr (kPlain) {
+        const double y = recip_refine(nz, inv);
+        sx += div_plain(nx, nz, y);                  // the sign of a zero term is lost in
+        sy += div_plain(ny, nz, y);                  // sums that start from +0
+    } else {
+        sx += nx/nz;
+        sy += ny/nz;
+    }
 }
 
-BT_DEV void sum_normal_from_slopes(double sx, double sy, double& nx, double& ny, double& nz)
+template <bool kPlain>
+BT_DEV void sum_normal_from_slopes(double sx, double sy, double& nx, double& ny, double& nz,
+                                   Range& rg)
 {
-    nz = cr_rsqrt(sx*sx + sy*sy + 1);
+    const double w = sx*sx + sy*sy + 1;
+    if constexpr (kPlain) {
+        double root;
+        rg.above(__builtin_fmax(w, 1.0));            // a child's NaN slopes: a NaN normal
+        nz = rsqrt_plain(w, root);
+    } else {
+        nz = cr_rsqrt(w);
+    }
     nx = sx*nz;
     ny = sy*nz;
 }
@@ -559,261 +792,161 @@ BT_DEV void sum_normal_from_slopes(double sx, double sy, double& nx, double& ny,
 // (the host refuses deeper trees; a deeper child evaluates to NaN).
 constexpr int kMaxSumDepth = 3;
 
-BT_DEV const bt_surface* next_child(const bt_surface* c)
+BT_DEV SurfPtr next_child(SurfPtr c)
 {
     return c + (c->kind == BT_SUM ? 1 + c->n1 : 1);
 }
 
-template <int D>
-BT_DEV double sum_sag_all(const bt_surface* s, double x, double y)
-{                                                    // sum.cpp:23-28
-    double result = 0.0;
-    const bt_surface* c = s + 1;
+template <int D, bool kPlain, bool kSag, bool kNormal>
+BT_DEV void sum_point_all(SurfPtr s, double x, double y, double& sag,
+                          double& nx, double& ny, double& nz, Range& rg)
+{                                                    // sum.cpp:23-45
+    double result = 0.0, sx = 0.0, sy = 0.0, ts, tnx, tny, tnz, inv;
+    SurfPtr c = s + 1;
     const int nc = s->nchild;
     for (int i = 0; i < nc; i++, c = next_child(c)) {
         if (c->kind != BT_SUM) {
-            result += leaf_sag<kKindsAll>(c, x, y);
+            leaf_point<kKindsAll, kPlain, kSag, kNormal>(c, x, y, ts, tnx, tny, tnz, inv, rg);
         } else {
-            if constexpr (D > 0) result += sum_sag_all<D - 1>(c, x, y);
-            else result += __builtin_nan("");
-        }
-    }
-    return result;
-}
-
-template <int D>
-BT_DEV void sum_normal_all(const bt_surface* s, double x, double y,
-                           double& nx, double& ny, double& nz)
-{                                                    // sum.cpp:30-45
-    double sx = 0.0, sy = 0.0, tnx, tny, tnz;
-    const bt_surface* c = s + 1;
-    const int nc = s->nchild;
-    for (int i = 0; i < nc; i++, c = next_child(c)) {
-        if (c->kind != BT_SUM) {
-            leaf_normal<kKindsAll>(c, x, y, tnx, tny, tnz);
-        } else {
-            if constexpr (D > 0) sum_normal_all<D - 1>(c, x, y, tnx, tny, tnz);
-            else { tnx = __builtin_nan(""); tny = tnx; tnz = tnx; }
-        }
-        add_slope(sx, sy, tnx, tny, tnz);
-    }
-    sum_normal_from_slopes(sx, sy, nx, ny, nz);
-}
-
-template <int D>
-BT_DEV void sum_sag_normal_all(const bt_surface* s, double x, double y, double& sag,
-                               double& nx, double& ny, double& nz)
-{
-    double result = 0.0, sx = 0.0, sy = 0.0, ts, tnx, tny, tnz;
-    const bt_surface* c = s + 1;
-    const int nc = s->nchild;
-    for (int i = 0; i < nc; i++, c = next_child(c)) {
-        if (c->kind != BT_SUM) {
-            leaf_sag_normal<kKindsAll>(c, x, y, ts, tnx, tny, tnz);
-        } else {
-            if constexpr (D > 0) sum_sag_normal_all<D - 1>(c, x, y, ts, tnx, tny, tnz);
+            inv = 0.0;
+            if constexpr (D > 0)
+                sum_point_all<D - 1, kPlain, kSag, kNormal>(c, x, y, ts, tnx, tny, tnz, rg);
             else { ts = __builtin_nan(""); tnx = ts; tny = ts; tnz = ts; }
         }
-        result += ts;
-        add_slope(sx, sy, tnx, tny, tnz);
+        if constexpr (kSag) result += ts;
+        if constexpr (kNormal) add_slope<kPlain>(sx, sy, tnx, tny, tnz, inv);
     }
-    sag = result;
-    sum_normal_from_slopes(sx, sy, nx, ny, nz);
+    if constexpr (kSag) sag = result;
+    if constexpr (kNormal) sum_normal_from_slopes<kPlain>(sx, sy, nx, ny, nz, rg);
+}
+
+// A Sum whose layout sum_is_apb has accepted.
+template <bool kPlain, bool kSag, bool kNormal>
+BT_DEV void apb_point(SurfPtr s, double x, double y, double& sag,
+                      double& nx, double& ny, double& nz, Range& rg)
+{
+    double result = 0.0, sx = 0.0, sy = 0.0, ts, tnx, tny, tnz, inv;
+    conic_point<kPlain, true, kSag, kNormal>(s + 1, x, y, ts, tnx, tny, tnz, inv, rg);
+    if constexpr (kSag) result += ts;
+    if constexpr (kNormal) add_slope<kPlain>(sx, sy, tnx, tny, tnz, inv);
+    if constexpr (kSag) result += poly_sag(s + 2, x, y);
+    if constexpr (kNormal) {
+        poly_normal<kPlain>(s + 2, x, y, tnx, tny, tnz, inv, rg);
+        add_slope<kPlain>(sx, sy, tnx, tny, tnz, inv);
+    }
+    table_point<kPlain, kSag, kNormal>(s + 3, x, y, ts, tnx, tny, tnz, inv, rg);
+    if constexpr (kSag) sag = result + ts;
+    if constexpr (kNormal) {
+        add_slope<kPlain>(sx, sy, tnx, tny, tnz, inv);
+        sum_normal_from_slopes<kPlain>(sx, sy, nx, ny, nz, rg);
+    }
 }
 
 // Sum records are followed by their children (sum.cpp:23-45).  The Sum's
 // sag is 0 + child sags in child order, its normal from the sum of the
 // children's slopes (-n_x/n_z, -n_y/n_z) in child order, so the unrolled
-// kKindsSumAPB forms below are the same operations as the loops.
-template <int K = kKindsAll>
-BT_DEV double surf_sag(const bt_surface* s, double x, double y)
+// kKindsSumAPB form is the same operations as the loops.
+template <int K, bool kPlain, bool kSag, bool kNormal>
+BT_DEV void surf_point(SurfPtr s, double x, double y, double& sag,
+                       double& nx, double& ny, double& nz, Range& rg)
 {
     constexpr int L = leaf_set(K);
-    if (K == kKindsAnalytic || s->kind != BT_SUM) return leaf_sag<L>(s, x, y);
-    double result = 0.0;
+    double inv;
+    if (K == kKindsAnalytic || s->kind != BT_SUM) {
+        leaf_point<L, kPlain, kSag, kNormal>(s, x, y, sag, nx, ny, nz, inv, rg);
+        return;
+    }
     if constexpr (K == kKindsSumAPB) {
-        if (!sum_is_apb(s)) return __builtin_nan("");
-        result += asphere_sag(s + 1, x, y);
-        result += poly_sag(s + 2, x, y);
-        result += table_eval(s + 3, x, y);
-        return result;
+        if (sum_is_apb(s)) {
+            apb_point<kPlain, kSag, kNormal>(s, x, y, sag, nx, ny, nz, rg);
+        } else {
+            const double nan = __builtin_nan("");
+            if constexpr (kSag) sag = nan;
+            if constexpr (kNormal) { nx = nan; ny = nan; nz = nan; }
+        }
     } else if constexpr (K == kKindsFlatSums) {
+        double result = 0.0, sx = 0.0, sy = 0.0, ts, tnx, tny, tnz;
         const int nc = s->nchild;
-        for (int i = 0; i < nc; i++)
-            result += leaf_sag<L>(s + 1 + i, x, y);
-        return result;
-    } else {
-        return sum_sag_all<kMaxSumDepth>(s, x, y);
+        for (int i = 0; i < nc; i++) {
+            leaf_point<L, kPlain, kSag, kNormal>(s + 1 + i, x, y, ts, tnx, tny, tnz, inv, rg);
+            if constexpr (kSag) result += ts;
+            if constexpr (kNormal) add_slope<kPlain>(sx, sy, tnx, tny, tnz, inv);
+        }
+        if constexpr (kSag) sag = result;
+        if constexpr (kNormal) sum_normal_from_slopes<kPlain>(sx, sy, nx, ny, nz, rg);
+    } else if constexpr (K == kKindsAll) {
+        sum_point_all<kMaxSumDepth, kPlain, kSag, kNormal>(s, x, y, sag, nx, ny, nz, rg);
     }
 }
 
+// Sag alone and normal alone, for callers without an interaction's vote.
 template <int K = kKindsAll>
-BT_DEV void surf_normal(const bt_surface* s, double x, double y,
+BT_DEV double surf_sag(SurfPtr s, double x, double y)
+{
+    double sag, nx, ny, nz;
+    Range rg;
+    surf_point<K, false, true, false>(s, x, y, sag, nx, ny, nz, rg);
+    return sag;
+}
+
+template <int K = kKindsAll>
+BT_DEV void surf_normal(SurfPtr s, double x, double y,
                         double& nx, double& ny, double& nz)
 {
-    constexpr int L = leaf_set(K);
-    if (K == kKindsAnalytic || s->kind != BT_SUM) { leaf_normal<L>(s, x, y, nx, ny, nz); return; }
-    double sx = 0.0, sy = 0.0;
-    double tnx, tny, tnz;
-    if constexpr (K == kKindsSumAPB) {
-        if (!sum_is_apb(s)) { nx = __builtin_nan(""); ny = nx; nz = nx; return; }
-        conic_normal<true>(s + 1, x, y, tnx, tny, tnz);
-        add_slope(sx, sy, tnx, tny, tnz);
-        poly_normal(s + 2, x, y, tnx, tny, tnz);
-        add_slope(sx, sy, tnx, tny, tnz);
-        table_normal(s + 3, x, y, tnx, tny, tnz);
-        add_slope(sx, sy, tnx, tny, tnz);
-        sum_normal_from_slopes(sx, sy, nx, ny, nz);
-        return;
-    } else if constexpr (K == kKindsFlatSums) {
-        const int nc = s->nchild;
-        for (int i = 0; i < nc; i++) {
-            leaf_normal<L>(s + 1 + i, x, y, tnx, tny, tnz);
-            add_slope(sx, sy, tnx, tny, tnz);
-        }
-        sum_normal_from_slopes(sx, sy, nx, ny, nz);
-    } else {
-        sum_normal_all<kMaxSumDepth>(s, x, y, nx, ny, nz);
-    }
-}
-
-template <int K = kKindsAll>
-BT_DEV void surf_sag_normal(const bt_surface* s, double x, double y, double& sag,
-                            double& nx, double& ny, double& nz)
-{
-    constexpr int L = leaf_set(K);
-    if (K == kKindsAnalytic || s->kind != BT_SUM) {
-        leaf_sag_normal<L>(s, x, y, sag, nx, ny, nz);
-        return;
-    }
-    double result = 0.0, sx = 0.0, sy = 0.0;
-    double ts, tnx, tny, tnz;
-    if constexpr (K == kKindsSumAPB) {
-        if (!sum_is_apb(s)) { sag = __builtin_nan(""); nx = sag; ny = sag; nz = sag; return; }
-        result += asphere_sag(s + 1, x, y);
-        conic_normal<true>(s + 1, x, y, tnx, tny, tnz);
-        add_slope(sx, sy, tnx, tny, tnz);
-        result += poly_sag(s + 2, x, y);
-        poly_normal(s + 2, x, y, tnx, tny, tnz);
-        add_slope(sx, sy, tnx, tny, tnz);
-        table_sag_normal(s + 3, x, y, ts, tnx, tny, tnz);
-        result += ts;
-        add_slope(sx, sy, tnx, tny, tnz);
-        sag = result;
-        sum_normal_from_slopes(sx, sy, nx, ny, nz);
-        return;
-    } else if constexpr (K == kKindsFlatSums) {
-        const int nc = s->nchild;
-        for (int i = 0; i < nc; i++) {
-            leaf_sag_normal<L>(s + 1 + i, x, y, ts, tnx, tny, tnz);
-            result += ts;
-            add_slope(sx, sy, tnx, tny, tnz);
-        }
-        sag = result;
-        sum_normal_from_slopes(sx, sy, nx, ny, nz);
-    } else {
-        sum_sag_normal_all<kMaxSumDepth>(s, x, y, sag, nx, ny, nz);
-    }
+    double sag;
+    Range rg;
+    surf_point<K, false, false, true>(s, x, y, sag, nx, ny, nz, rg);
 }
 
 // Surface evaluators for the Newton loops.  SurfEval<K> dispatches on the
 // record's kind at every evaluation; where the caller already knows the kind
 // (an Asphere leaf, a Sum laid out as kKindsSumAPB requires) the loop is
 // instantiated with that kind's functions directly, so it carries no switch
-// over the other kinds.  Every evaluator computes exactly what surf_sag /
-// surf_normal / surf_sag_normal compute for that record.
+// over the other kinds.  Every evaluator computes exactly what surf_point
+// computes for that record.  kGrid: the record may hold a Bicubic, whose sag
+// is NaN off its grid.
 template <int K>
 struct SurfEval {
-    static BT_DEV double sag(const bt_surface* s, double x, double y)
+    static constexpr bool kGrid = K != kKindsAnalytic;
+    template <bool kPlain, bool kSag, bool kNormal>
+    static BT_DEV void point(SurfPtr s, double x, double y, double& sag,
+                             double& nx, double& ny, double& nz, Range& rg)
     {
-        return surf_sag<K>(s, x, y);
-    }
-    static BT_DEV void normal(const bt_surface* s, double x, double y, double& nx, double& ny,
-                              double& nz)
-    {
-        surf_normal<K>(s, x, y, nx, ny, nz);
-    }
-    static BT_DEV void sag_normal(const bt_surface* s, double x, double y, double& sag,
-                                  double& nx, double& ny, double& nz)
-    {
-        surf_sag_normal<K>(s, x, y, sag, nx, ny, nz);
+        surf_point<K, kPlain, kSag, kNormal>(s, x, y, sag, nx, ny, nz, rg);
     }
 };
 
 // A record known to be a leaf (not a Sum).
 template <int K>
 struct LeafEval {
-    static BT_DEV double sag(const bt_surface* s, double x, double y)
+    static constexpr bool kGrid = K == kKindsAll;
+    template <bool kPlain, bool kSag, bool kNormal>
+    static BT_DEV void point(SurfPtr s, double x, double y, double& sag,
+                             double& nx, double& ny, double& nz, Range& rg)
     {
-        return leaf_sag<K>(s, x, y);
-    }
-    static BT_DEV void normal(const bt_surface* s, double x, double y, double& nx, double& ny,
-                              double& nz)
-    {
-        leaf_normal<K>(s, x, y, nx, ny, nz);
-    }
-    static BT_DEV void sag_normal(const bt_surface* s, double x, double y, double& sag,
-                                  double& nx, double& ny, double& nz)
-    {
-        leaf_sag_normal<K>(s, x, y, sag, nx, ny, nz);
+        double inv;
+        leaf_point<K, kPlain, kSag, kNormal>(s, x, y, sag, nx, ny, nz, inv, rg);
     }
 };
 
 struct AsphereEval {                                 // asphere.cpp:37-62
-    static BT_DEV double sag(const bt_surface* s, double x, double y)
+    static constexpr bool kGrid = false;
+    template <bool kPlain, bool kSag, bool kNormal>
+    static BT_DEV void point(SurfPtr s, double x, double y, double& sag,
+                             double& nx, double& ny, double& nz, Range& rg)
     {
-        return asphere_sag(s, x, y);
-    }
-    static BT_DEV void normal(const bt_surface* s, double x, double y, double& nx, double& ny,
-                              double& nz)
-    {
-        conic_normal<true>(s, x, y, nx, ny, nz);
-    }
-    static BT_DEV void sag_normal(const bt_surface* s, double x, double y, double& sag,
-                                  double& nx, double& ny, double& nz)
-    {
-        sag = asphere_sag(s, x, y);
-        conic_normal<true>(s, x, y, nx, ny, nz);
+        double inv;
+        conic_point<kPlain, true, kSag, kNormal>(s, x, y, sag, nx, ny, nz, inv, rg);
     }
 };
 
-// A Sum whose layout sum_is_apb has accepted (sum.cpp:23-45).
-struct SumAPBEval {
-    static BT_DEV double sag(const bt_surface* s, double x, double y)
+struct SumAPBEval {                                  // sum.cpp:23-45
+    static constexpr bool kGrid = true;
+    template <bool kPlain, bool kSag, bool kNormal>
+    static BT_DEV void point(SurfPtr s, double x, double y, double& sag,
+                             double& nx, double& ny, double& nz, Range& rg)
     {
-        double result = 0.0;
-        result += asphere_sag(s + 1, x, y);
-        result += poly_sag(s + 2, x, y);
-        result += table_eval(s + 3, x, y);
-        return result;
-    }
-    static BT_DEV void normal(const bt_surface* s, double x, double y, double& nx, double& ny,
-                              double& nz)
-    {
-        double sx = 0.0, sy = 0.0, tnx, tny, tnz;
-        conic_normal<true>(s + 1, x, y, tnx, tny, tnz);
-        add_slope(sx, sy, tnx, tny, tnz);
-        poly_normal(s + 2, x, y, tnx, tny, tnz);
-        add_slope(sx, sy, tnx, tny, tnz);
-        table_normal(s + 3, x, y, tnx, tny, tnz);
-        add_slope(sx, sy, tnx, tny, tnz);
-        sum_normal_from_slopes(sx, sy, nx, ny, nz);
-    }
-    static BT_DEV void sag_normal(const bt_surface* s, double x, double y, double& sag,
-                                  double& nx, double& ny, double& nz)
-    {
-        double result = 0.0, sx = 0.0, sy = 0.0, ts, tnx, tny, tnz;
-        result += asphere_sag(s + 1, x, y);
-        conic_normal<true>(s + 1, x, y, tnx, tny, tnz);
-        add_slope(sx, sy, tnx, tny, tnz);
-        result += poly_sag(s + 2, x, y);
-        poly_normal(s + 2, x, y, tnx, tny, tnz);
-        add_slope(sx, sy, tnx, tny, tnz);
-        table_sag_normal(s + 3, x, y, ts, tnx, tny, tnz);
-        result += ts;
-        add_slope(sx, sy, tnx, tny, tnz);
-        sag = result;
-        sum_normal_from_slopes(sx, sy, nx, ny, nz);
+        apb_point<kPlain, kSag, kNormal>(s, x, y, sag, nx, ny, nz, rg);
     }
 };
 
@@ -830,45 +963,71 @@ BT_DEV bool same_bits(double a, double b)
 // neighbouring doubles dt'' == dt -- every remaining iterate is known, and the
 // loop stops with exactly the state (dt, rP, sag) that running all `niter`
 // iterations would leave.  Results are bit-identical to the full loop.
-// The last surface normal Newton evaluated and the dt of the point it was
-// evaluated at: a reflection or refraction at that same point reuses it
-// (surf_normal of bit-identical arguments is bit-identical).
-struct NormalMemo {
+//
+struct NormalMemo {              // the normal at the ray's point at dt
     double dt, nx, ny, nz;
     bool ok;
 };
 
-template <class Ev>
-BT_DEV bool newton(const bt_surface* s, double x, double y, double z,
-                   double vx, double vy, double vz, double& dt, int niter,
+// The plain form evaluates sag and normal together at each iterate (roots'
+// arguments, table cells and coefficient loads shared) and leaves the final
+// point's normal for the reflection or refraction there.  The full form
+// evaluates them apart, which needs fewer registers; its memo is the last
+// normal evaluated, used where it belongs to the final point.
+template <class Ev, bool kPlain>
+BT_DEV bool newton(SurfPtr s, double x, double y, double z,
+                   double vx, double vy, double vz, double& dt, int niter, Range& rg,
                    NormalMemo* memo = nullptr)
 {
-    double rPx = x+vx*dt;
-    double rPy = y+vy*dt;
-    double rPz = z+vz*dt;
-    double sz = Ev::sag(s, rPx, rPy);
+    double nx, ny, nz, sz, rPz, unused;
     double pdt = 0.0;            // the iterate before the current one (iter >= 1)
-    for (int iter = 0; iter < niter; iter++) {
-        double nx, ny, nz;
-        Ev::normal(s, rPx, rPy, nx, ny, nz);
-        if (memo) *memo = NormalMemo{dt, nx, ny, nz, true};
-        double dtn = (rPx-x)*nx + (rPy-y)*ny + (sz-z)*nz;
-        dtn /= (nx*vx + ny*vy + nz*vz);
-        if (same_bits(dtn, dt)) break;            // fixed point: state unchanged
-        const double odt = dt, oz = rPz, osz = sz;
-        dt = dtn;
-        rPx = x+vx*dt;
-        rPy = y+vy*dt;
-        rPz = z+vz*dt;
-        sz = Ev::sag(s, rPx, rPy);
-        if (iter >= 1 && same_bits(dt, pdt)) {
-            // two-cycle: iterates alternate between this state and the
-            // previous one; after the remaining (niter-1-iter) iterations the
-            // loop ends on this state if that count is even, else on the other
-            if ((niter - 1 - iter) & 1) { dt = odt; rPz = oz; sz = osz; }
-            break;
+    if constexpr (kPlain) {
+        bool last = niter <= 0;  // nothing is iterated from the current point
+        for (int iter = 0;; iter++) {
+            const double rPx = x+vx*dt;
+            const double rPy = y+vy*dt;
+            rPz = z+vz*dt;
+            Ev::template point<true, true, true>(s, rPx, rPy, sz, nx, ny, nz, rg);
+            if (last) break;
+            double dtn = (rPx-x)*nx + (rPy-y)*ny + (sz-z)*nz;
+            dtn /= (nx*vx + ny*vy + nz*vz);
+            if (same_bits(dtn, dt)) break;        // fixed point: state unchanged
+            // off a Bicubic's grid: every later iterate is NaN, and the ray
+            // fails
+            if (Ev::kGrid && !(dtn == dtn)) { sz = dtn; break; }
+            // two-cycle: iterates alternate between the next point and this
+            // one; the remaining niter-1-iter iterations end on the next
+            // point if that count is even, else here
+            const bool cycle = iter >= 1 && same_bits(dtn, pdt);
+            if (cycle && ((niter - 1 - iter) & 1)) break;
+            last = cycle || iter + 1 >= niter;
+            pdt = dt;
+            dt = dtn;
         }
-        pdt = odt;
+        if (memo) *memo = NormalMemo{dt, nx, ny, nz, true};
+    } else {
+        double rPx = x+vx*dt;
+        double rPy = y+vy*dt;
+        rPz = z+vz*dt;
+        Ev::template point<false, true, false>(s, rPx, rPy, sz, unused, unused, unused, rg);
+        for (int iter = 0; iter < niter; iter++) {
+            Ev::template point<false, false, true>(s, rPx, rPy, unused, nx, ny, nz, rg);
+            if (memo) *memo = NormalMemo{dt, nx, ny, nz, true};
+            double dtn = (rPx-x)*nx + (rPy-y)*ny + (sz-z)*nz;
+            dtn /= (nx*vx + ny*vy + nz*vz);
+            if (same_bits(dtn, dt)) break;
+            const double odt = dt, oz = rPz, osz = sz;
+            dt = dtn;
+            rPx = x+vx*dt;
+            rPy = y+vy*dt;
+            rPz = z+vz*dt;
+            Ev::template point<false, true, false>(s, rPx, rPy, sz, unused, unused, unused, rg);
+            if (iter >= 1 && same_bits(dt, pdt)) {
+                if ((niter - 1 - iter) & 1) { dt = odt; rPz = oz; sz = osz; }
+                break;
+            }
+            pdt = odt;
+        }
     }
     return fabs(sz-rPz) < 1e-12;
 }
@@ -880,8 +1039,9 @@ BT_DEV double pick_root(double vzR, double dt1, double dt2)
     return (dt2 < dt1) ? dt2 : dt1;
 }
 
-BT_DEV bool quadric_tti(const bt_surface* s, double x, double y, double z,
-                        double vx, double vy, double vz, double& dt)
+template <bool kPlain>
+BT_DEV bool quadric_tti(SurfPtr s, double x, double y, double z,
+                        double vx, double vy, double vz, double& dt, Range& rg)
 {                                                    // quadric.cpp:41-70
     double z0term = z-s->p[6];
     double vrr0 = vx*x + vy*y;
@@ -891,11 +1051,12 @@ BT_DEV bool quadric_tti(const bt_surface* s, double x, double y, double z,
     double discriminant = b*b - 4*a*c;
     if (discriminant < 0)
         return false;
+    const double root = root_of<kPlain>(discriminant, rg);
     double dt1;
     if (b > 0)
-        dt1 = (-b - cr_sqrt(discriminant)) / (2*a);
+        dt1 = (-b - root) / (2*a);
     else
-        dt1 = 2*c / (-b + cr_sqrt(discriminant));
+        dt1 = 2*c / (-b + root);
     double dt2 = c / (a*dt1);
     double z1 = z + vz*dt1;
     double z2 = z + vz*dt2;
@@ -903,9 +1064,9 @@ BT_DEV bool quadric_tti(const bt_surface* s, double x, double y, double z,
     return true;
 }
 
-template <int K = kKindsAll>
-BT_DEV bool leaf_tti(const bt_surface* s, double x, double y, double z,
-                     double vx, double vy, double vz, double& dt, int niter,
+template <int K, bool kPlain>
+BT_DEV bool leaf_tti(SurfPtr s, double x, double y, double z,
+                     double vx, double vy, double vz, double& dt, int niter, Range& rg,
                      NormalMemo* memo = nullptr)
 {
     switch (s->kind) {
@@ -925,11 +1086,12 @@ BT_DEV bool leaf_tti(const bt_surface* s, double x, double y, double z,
         double c = z0term*z0term - s->p[1] + r02;
         double discriminant = b*b - 4*a*c;
         if (discriminant < 0) return false;
+        const double root = root_of<kPlain>(discriminant, rg);
         double dt1;
         if (b > 0)
-            dt1 = (-b - cr_sqrt(discriminant)) / (2*a);
+            dt1 = (-b - root) / (2*a);
         else
-            dt1 = 2*c / (-b + cr_sqrt(discriminant));
+            dt1 = 2*c / (-b + root);
         double dt2 = c / (a*dt1);
         dt = pick_root(vz*R, dt1, dt2);
         return true;
@@ -944,20 +1106,21 @@ BT_DEV bool leaf_tti(const bt_surface* s, double x, double y, double z,
         }
         double discriminant = b*b - 4*a*c;
         if (discriminant < 0) return false;
+        const double root = root_of<kPlain>(discriminant, rg);
         double dt1;
         if (b > 0)
-            dt1 = (-b - cr_sqrt(discriminant)) / (2*a);
+            dt1 = (-b - root) / (2*a);
         else
-            dt1 = 2*c / (-b + cr_sqrt(discriminant));
+            dt1 = 2*c / (-b + root);
         double dt2 = c / (a*dt1);
         dt = pick_root(vz*s->p[0], dt1, dt2);
         return true;
     }
     case BT_QUADRIC:
-        return quadric_tti(s, x, y, z, vx, vy, vz, dt);
+        return quadric_tti<kPlain>(s, x, y, z, vx, vy, vz, dt, rg);
     case BT_ASPHERE:                                 // asphere.cpp:75-85
-        if (!quadric_tti(s, x, y, z, vx, vy, vz, dt)) return false;
-        return newton<AsphereEval>(s, x, y, z, vx, vy, vz, dt, niter, memo);
+        if (!quadric_tti<kPlain>(s, x, y, z, vx, vy, vz, dt, rg)) return false;
+        return newton<AsphereEval, kPlain>(s, x, y, z, vx, vy, vz, dt, niter, rg, memo);
     case BT_TILTED: {                                // tilted.cpp:29-37
         double num = z - x*s->p[0] - y*s->p[1];
         double den = vx*s->p[0] + vy*s->p[1] - vz;
@@ -968,7 +1131,7 @@ BT_DEV bool leaf_tti(const bt_surface* s, double x, double y, double z,
     case BT_BICUBIC:
     case BT_POLYNOMIAL:                              // surface.cpp:22-49
         if constexpr (K == kKindsAll)
-            return newton<LeafEval<K>>(s, x, y, z, vx, vy, vz, dt, niter, memo);
+            return newton<LeafEval<K>, kPlain>(s, x, y, z, vx, vy, vz, dt, niter, rg, memo);
         break;
     }
     return false;
@@ -976,69 +1139,70 @@ BT_DEV bool leaf_tti(const bt_surface* s, double x, double y, double z,
 
 // sum.cpp:47-56: the first child's intersection (itself a Sum's, to the
 // nesting depth kKindsAll allows) seeds Newton on the Sum.
-template <int D>
-BT_DEV bool sum_tti_all(const bt_surface* s, double x, double y, double z,
-                        double vx, double vy, double vz, double& dt, int niter,
+template <int D, bool kPlain>
+BT_DEV bool sum_tti_all(SurfPtr s, double x, double y, double z,
+                        double vx, double vy, double vz, double& dt, int niter, Range& rg,
                         NormalMemo* memo)
 {
-    const bt_surface* c = s + 1;
-    bool ok = false;
+    SurfPtr c = s + 1;
+    bool hit = false;
     if (c->kind != BT_SUM) {
-        ok = leaf_tti<kKindsAll>(c, x, y, z, vx, vy, vz, dt, niter);
+        hit = leaf_tti<kKindsAll, kPlain>(c, x, y, z, vx, vy, vz, dt, niter, rg);
     } else {
-        if constexpr (D > 0) ok = sum_tti_all<D - 1>(c, x, y, z, vx, vy, vz, dt, niter, nullptr);
+        if constexpr (D > 0)
+            hit = sum_tti_all<D - 1, kPlain>(c, x, y, z, vx, vy, vz, dt, niter, rg, nullptr);
     }
-    if (!ok) return false;
-    return newton<SurfEval<kKindsAll>>(s, x, y, z, vx, vy, vz, dt, niter, memo);
+    if (!hit) return false;
+    return newton<SurfEval<kKindsAll>, kPlain>(s, x, y, z, vx, vy, vz, dt, niter, rg, memo);
 }
 
-template <int K = kKindsAll>
-BT_DEV bool surf_tti(const bt_surface* s, double x, double y, double z,
-                     double vx, double vy, double vz, double& dt, int niter,
+template <int K, bool kPlain>
+BT_DEV bool surf_tti(SurfPtr s, double x, double y, double z,
+                     double vx, double vy, double vz, double& dt, int niter, Range& rg,
                      NormalMemo* memo = nullptr)
 {
     constexpr int L = leaf_set(K);
     if (K == kKindsAnalytic || s->kind != BT_SUM)
-        return leaf_tti<L>(s, x, y, z, vx, vy, vz, dt, niter, memo);
+        return leaf_tti<L, kPlain>(s, x, y, z, vx, vy, vz, dt, niter, rg, memo);
     if constexpr (K == kKindsSumAPB) {
         if (!sum_is_apb(s)) return false;
-        if (!leaf_tti<L>(s + 1, x, y, z, vx, vy, vz, dt, niter)) return false;
-        return newton<SumAPBEval>(s, x, y, z, vx, vy, vz, dt, niter, memo);
+        if (!leaf_tti<L, kPlain>(s + 1, x, y, z, vx, vy, vz, dt, niter, rg)) return false;
+        return newton<SumAPBEval, kPlain>(s, x, y, z, vx, vy, vz, dt, niter, rg, memo);
     } else if constexpr (K == kKindsFlatSums) {
-        if (!leaf_tti<L>(s + 1, x, y, z, vx, vy, vz, dt, niter)) return false;
-        return newton<SurfEval<K>>(s, x, y, z, vx, vy, vz, dt, niter, memo);
+        if (!leaf_tti<L, kPlain>(s + 1, x, y, z, vx, vy, vz, dt, niter, rg)) return false;
+        return newton<SurfEval<K>, kPlain>(s, x, y, z, vx, vy, vz, dt, niter, rg, memo);
     } else {
-        return sum_tti_all<kMaxSumDepth>(s, x, y, z, vx, vy, vz, dt, niter, memo);
+        return sum_tti_all<kMaxSumDepth, kPlain>(s, x, y, z, vx, vy, vz, dt, niter, rg, memo);
     }
 }
 
 // The surface's analytic base start: the root of a Sum's first child or of an
 // Asphere's conic (the starts of sum.cpp:53 and asphere.cpp:82, without the
 // Newton refinement that follows them); surfaces without one start at 0.
-template <int K = kKindsAll>
-BT_DEV bool conic_start(const bt_surface* s, double x, double y, double z, double vx,
-                        double vy, double vz, double& dt)
+template <int K, bool kPlain>
+BT_DEV bool conic_start(SurfPtr s, double x, double y, double z, double vx,
+                        double vy, double vz, double& dt, Range& rg)
 {
-    const bt_surface* c = s;
+    SurfPtr c = s;
     if (K != kKindsAnalytic)
         while (c->kind == BT_SUM) c = c + 1;     // the first leaf of nested Sums
     dt = 0.0;
     switch (c->kind) {
     case BT_ASPHERE:
     case BT_QUADRIC:
-        return quadric_tti(c, x, y, z, vx, vy, vz, dt);
+        return quadric_tti<kPlain>(c, x, y, z, vx, vy, vz, dt, rg);
     case BT_PLANE:
     case BT_SPHERE:
     case BT_PARABOLOID:
     case BT_TILTED:
-        return leaf_tti<leaf_set(K)>(c, x, y, z, vx, vy, vz, dt, 0);
+        return leaf_tti<leaf_set(K), kPlain>(c, x, y, z, vx, vy, vz, dt, 0, rg);
     default:
         return true;
     }
 }
 
 
-BT_DEV bool newton_surface(const bt_surface* s)
+BT_DEV bool newton_surface(SurfPtr s)
 {
     return s->kind == BT_SUM || s->kind == BT_ASPHERE || s->kind == BT_BICUBIC ||
            s->kind == BT_POLYNOMIAL;
@@ -1053,22 +1217,23 @@ constexpr double kFastTol = 1e-14;   // sag gap accepted by the fast starts [m]
 // the reference path, which decides it).  At 1e-13 m the residual position
 // errors, carried through a three-mirror optic, reach ~1e-14 in the final
 // direction cosines; 1e-14 m keeps them an order of magnitude below that.
-template <class Ev>
-BT_DEV bool newton_fast(const bt_surface* s, double x, double y, double z,
+template <class Ev, bool kPlain>
+BT_DEV bool newton_fast(SurfPtr s, double x, double y, double z,
                         double vx, double vy, double vz, double& dt, NormalMemo* memo,
-                        int max_iter)
+                        int max_iter, Range& rg)
 {
     double rPx = x+vx*dt, rPy = y+vy*dt, rPz = z+vz*dt;
     double sz, nx, ny, nz;
-    Ev::sag_normal(s, rPx, rPy, sz, nx, ny, nz);
+    Ev::template point<kPlain, true, true>(s, rPx, rPy, sz, nx, ny, nz, rg);
     for (int it = 0; it < max_iter; it++) {
         if (fabs(sz-rPz) <= kFastTol) break;
         double d = (rPx-x)*nx + (rPy-y)*ny + (sz-z)*nz;
         dt = d / (nx*vx + ny*vy + nz*vz);
+        if (Ev::kGrid && !(dt == dt)) return false;
         rPx = x+vx*dt;
         rPy = y+vy*dt;
         rPz = z+vz*dt;
-        Ev::sag_normal(s, rPx, rPy, sz, nx, ny, nz);
+        Ev::template point<kPlain, true, true>(s, rPx, rPy, sz, nx, ny, nz, rg);
     }
     if (!(fabs(sz-rPz) <= kFastTol)) return false;
     *memo = NormalMemo{dt, nx, ny, nz, true};
@@ -1077,12 +1242,13 @@ BT_DEV bool newton_fast(const bt_surface* s, double x, double y, double z,
 
 // One Newton update of `dt` on an Asphere alone (its sag and normal at the
 // ray's point at `dt`); `dt` is kept where the update is not finite.
-BT_DEV void asphere_update(const bt_surface* c, double x, double y, double z, double vx,
-                           double vy, double vz, double& dt)
+template <bool kPlain>
+BT_DEV void asphere_update(SurfPtr c, double x, double y, double z, double vx,
+                           double vy, double vz, double& dt, Range& rg)
 {
     const double rPx = x+vx*dt, rPy = y+vy*dt;
     double sz, nx, ny, nz;
-    AsphereEval::sag_normal(c, rPx, rPy, sz, nx, ny, nz);
+    AsphereEval::point<kPlain, true, true>(c, rPx, rPy, sz, nx, ny, nz, rg);
     const double d = (rPx-x)*nx + (rPy-y)*ny + (sz-z)*nz;
     const double t = d / (nx*vx + ny*vy + nz*vz);
     if (t == t) dt = t;
@@ -1101,37 +1267,38 @@ BT_DEV void asphere_update(const bt_surface* c, double x, double y, double z, do
 //   no conic base) plus `correction` (the network's prediction for
 //   BT_START_MLP, 0 for BT_START_CONIC).
 // The reference path decides every ray the fast start does not settle.
-template <int K = kKindsAll>
-BT_DEV bool fast_tti(const bt_surface* s, double x, double y, double z, double vx,
+template <int K, bool kPlain>
+BT_DEV bool fast_tti(SurfPtr s, double x, double y, double z, double vx,
                      double vy, double vz, double& dt, int niter, double correction,
-                     NormalMemo* memo)
+                     Range& rg, NormalMemo* memo)
 {
     if (newton_surface(s)) {
         double d0 = 0.0;
-        bool ok;
+        bool start;
         if (K != kKindsAnalytic && correction == 0.0 && s->kind == BT_SUM) {
-            const bt_surface* c = s + 1;
+            SurfPtr c = s + 1;
             if (c->kind == BT_ASPHERE) {
-                ok = quadric_tti(c, x, y, z, vx, vy, vz, d0);
-                if (ok) asphere_update(c, x, y, z, vx, vy, vz, d0);
+                start = quadric_tti<kPlain>(c, x, y, z, vx, vy, vz, d0, rg);
+                if (start) asphere_update<kPlain>(c, x, y, z, vx, vy, vz, d0, rg);
             } else if constexpr (K != kKindsSumAPB) {
-                ok = surf_tti<K>(c, x, y, z, vx, vy, vz, d0, niter);
+                start = surf_tti<K, kPlain>(c, x, y, z, vx, vy, vz, d0, niter, rg);
             } else {
-                ok = false;                     // not a Sum(Asphere, Polynomial, Bicubic)
+                start = false;                  // not a Sum(Asphere, Polynomial, Bicubic)
             }
         } else {
-            ok = conic_start<K>(s, x, y, z, vx, vy, vz, d0);
+            start = conic_start<K, kPlain>(s, x, y, z, vx, vy, vz, d0, rg);
             d0 += correction;
         }
         bool conv = false;
-        if (ok && d0 == d0) {
+        if (start && d0 == d0) {
             if (s->kind == BT_ASPHERE)
-                conv = newton_fast<AsphereEval>(s, x, y, z, vx, vy, vz, d0, memo, niter);
+                conv = newton_fast<AsphereEval, kPlain>(s, x, y, z, vx, vy, vz, d0, memo, niter, rg);
             else if constexpr (K == kKindsSumAPB)
                 conv = sum_is_apb(s) &&
-                       newton_fast<SumAPBEval>(s, x, y, z, vx, vy, vz, d0, memo, niter);
+                       newton_fast<SumAPBEval, kPlain>(s, x, y, z, vx, vy, vz, d0, memo, niter,
+                                                       rg);
             else
-                conv = newton_fast<SurfEval<K>>(s, x, y, z, vx, vy, vz, d0, memo, niter);
+                conv = newton_fast<SurfEval<K>, kPlain>(s, x, y, z, vx, vy, vz, d0, memo, niter, rg);
         }
         if (conv) {
             dt = d0;
@@ -1139,20 +1306,20 @@ BT_DEV bool fast_tti(const bt_surface* s, double x, double y, double z, double v
         }
     }
     dt = 0.0;
-    return surf_tti<K>(s, x, y, z, vx, vy, vz, dt, niter, memo);
+    return surf_tti<K, kPlain>(s, x, y, z, vx, vy, vz, dt, niter, rg, memo);
 }
 
 // ---------------------------------------------------------------------------
 // Media (src/medium.cpp)
 // ---------------------------------------------------------------------------
-BT_DEV double medium_n(const bt_medium* m, double w)
+BT_DEV double medium_n(MediumPtr m, double w)
 {
     switch (m->kind) {
     case BT_MED_CONST:                               // medium.cpp:30-32
         return m->p[0];
     case BT_MED_TABLE: {                             // medium.cpp:89-105
-        const double* __restrict__ args = m->a0;
-        const double* __restrict__ vals = m->a1;
+        const TablePtr args = (TablePtr)m->a0;
+        const TablePtr vals = (TablePtr)m->a1;
         const int size = m->n;
         if (w < args[0]) return __builtin_nan("");
         if (w > args[size-1]) return __builtin_nan("");
@@ -1166,12 +1333,12 @@ BT_DEV double medium_n(const bt_medium* m, double w)
         return out;
     }
     case BT_MED_SELLMEIER: {                         // medium.cpp:145-149
-        const double* p = m->p;
+        const CoefPtr p = m->p;
         double x = w*w*1e12;
         return cr_sqrt(1.0 + p[0]*x/(x-p[3]) + p[1]*x/(x-p[4]) + p[2]*x/(x-p[5]));
     }
     case BT_MED_SUMITA: {                            // medium.cpp:186-191
-        const double* A = m->p;
+        const CoefPtr A = m->p;
         double x = w*w*1e12;
         double y = 1./x;
         return cr_sqrt(A[0] + A[1]*x + y*(A[2] + y*(A[3] + y*(A[4] + y*A[5]))));
@@ -1266,10 +1433,10 @@ BT_DEV int cmp_hypot(double x, double y, double r)
 // ---------------------------------------------------------------------------
 // Obscuration programs (src/obscuration.cpp); the stack is a bit mask.
 // ---------------------------------------------------------------------------
-BT_DEV bool polygon_contains(const bt_obsc* o, double x, double y)
+BT_DEV bool polygon_contains(ObscPtr o, double x, double y)
 {                                                    // obscuration.cpp:201-225
-    const double* __restrict__ xp = o->a0;
-    const double* __restrict__ yp = o->a1;
+    const CoefPtr xp = (CoefPtr)o->a0;
+    const CoefPtr yp = (CoefPtr)o->a1;
     const int size = o->n;
     double x1 = xp[0];
     double y1 = yp[0];
@@ -1294,13 +1461,13 @@ BT_DEV bool polygon_contains(const bt_obsc* o, double x, double y)
     return inside;
 }
 
-BT_DEV bool obsc_contains(const bt_obsc* prog, int len, double x, double y)
+BT_DEV bool obsc_contains(ObscPtr prog, int len, double x, double y)
 {
     uint32_t stack = 0;   // bit k = stack slot k
     int sp = 0;
     for (int k = 0; k < len; k++) {
-        const bt_obsc* o = prog + k;
-        const double* p = o->p;
+        ObscPtr o = prog + k;
+        const CoefPtr p = o->p;
         bool v;
         switch (o->op) {
         case BT_OB_CIRCLE: {                         // obscuration.cpp:32-34
@@ -1366,113 +1533,260 @@ struct Ray {
     bool vig, fail;
 };
 
+// What a refraction and the reflected part of a split share at a surface of
+// normal n (batoid.cpp:453-470, 620-640): the incoming index n1 = 1/|v|, the
+// unit velocity nv, and the normal turned against it with alpha = nv.n <= 0.
+struct Incidence {
+    double n1, root, nvx, nvy, nvz, nx, ny, nz, alpha;
+};
+
+template <bool kPlain>
+BT_DEV Incidence incidence(double nx, double ny, double nz, double vx, double vy, double vz,
+                           Range& rg)
+{
+    Incidence c;
+    double n1 = vx*vx;
+    n1 += vy*vy;
+    n1 += vz*vz;
+    c.n1 = recip_root_of<kPlain>(n1, c.root, rg);
+    c.nvx = vx*c.n1;
+    c.nvy = vy*c.n1;
+    c.nvz = vz*c.n1;
+    double alpha = c.nvx*nx;
+    alpha += c.nvy*ny;
+    alpha += c.nvz*nz;
+    if (alpha > 0.) {
+        nx *= -1; ny *= -1; nz *= -1;
+        alpha *= -1;
+    }
+    c.nx = nx; c.ny = ny; c.nz = nz;
+    c.alpha = alpha;
+    return c;
+}
+
+// The velocity refracted into a medium of index n2 (batoid.cpp:474-496);
+// true for total internal reflection (NaN velocity).  Into a medium of index
+// exactly 1 (vacuum, or air given as a constant 1) the reference's divisions
+// by n2 return their numerators bit for bit (x/1 == x in IEEE arithmetic,
+// signed zeros, infinities and NaNs included), so that case runs without
+// them; into any other the plain form's four quotients share one reciprocal.
+template <bool kPlain>
+BT_DEV bool refract_velocity(const Incidence& c, double n2, double& vx, double& vy, double& vz,
+                             Range& rg)
+{
+    const bool unit = __all(n2 == 1.0);
+    double eta = c.n1, inv = 0.0;
+    if (!unit) {
+        if constexpr (kPlain) {
+            rg.positive(n2);
+            inv = recip_plain(n2);
+            eta = div_plain(c.n1, n2, inv);
+        } else {
+            eta /= n2;
+        }
+    }
+    const double sinsqr = eta*eta*(1-c.alpha*c.alpha);
+    if (sinsqr > 1.0) {
+        vx = __builtin_nan(""); vy = vx; vz = vx;
+        return true;
+    }
+    const double nfactor = eta*c.alpha + root_of<kPlain>(1-sinsqr, rg);
+    vx = eta*c.nvx - nfactor*c.nx;
+    vy = eta*c.nvy - nfactor*c.ny;
+    vz = eta*c.nvz - nfactor*c.nz;
+    if (!unit) {
+        if constexpr (kPlain) {
+            vx = div_plain_signed(vx, n2, inv);
+            vy = div_plain_signed(vy, n2, inv);
+            vz = div_plain_signed(vz, n2, inv);
+        } else {
+            vx /= n2;
+            vy /= n2;
+            vz /= n2;
+        }
+    }
+    return false;
+}
+
+// The velocity v - 2 alpha n / n1 of the reflected part of a split
+// (batoid.cpp:642-645), in place.
+template <bool kPlain>
+BT_DEV void split_reflect(const Incidence& c, double& vx, double& vy, double& vz, Range& rg)
+{
+    const double ax = 2*c.alpha*c.nx, ay = 2*c.alpha*c.ny, az = 2*c.alpha*c.nz;
+    if constexpr (kPlain) {
+        const double inv = recip_refine(c.n1, c.root);
+        vx = vx - div_plain_signed(ax, c.n1, inv);
+        vy = vy - div_plain_signed(ay, c.n1, inv);
+        vz = vz - div_plain_signed(az, c.n1, inv);
+    } else {
+        vx = vx - ax/c.n1;
+        vy = vy - ay/c.n1;
+        vz = vz - az/c.n1;
+    }
+}
+
+// A ray in an Interface's frame, advanced to its surface.
+struct Arrival {
+    double x, y, z, vx, vy, vz, t, dt;
+    NormalMemo memo;
+};
+
+// Frame change and intersection; false where the ray misses the surface.
+template <int K, bool kPlain, class Frame>
+BT_DEV bool arrive(Frame dr, Frame drot,
+                   SurfPtr surf, const Ray& r, int niter, int start,
+                   double correction, Arrival& a, Range& rg)
+{
+    double dx = r.x-dr[0];
+    double dy = r.y-dr[1];
+    double dz = r.z-dr[2];
+    a.x = dx*drot[0] + dy*drot[3] + dz*drot[6];
+    a.y = dx*drot[1] + dy*drot[4] + dz*drot[7];
+    a.z = dx*drot[2] + dy*drot[5] + dz*drot[8];
+    a.vx = r.vx*drot[0] + r.vy*drot[3] + r.vz*drot[6];
+    a.vy = r.vx*drot[1] + r.vy*drot[4] + r.vz*drot[7];
+    a.vz = r.vx*drot[2] + r.vy*drot[5] + r.vz*drot[8];
+    a.t = r.t;
+    a.dt = 0.0;
+    a.memo.ok = false;
+    const bool hit =
+        (start == BT_START_REFERENCE)
+            ? surf_tti<K, kPlain>(surf, a.x, a.y, a.z, a.vx, a.vy, a.vz, a.dt, niter, rg,
+                                  &a.memo)
+            : fast_tti<K, kPlain>(surf, a.x, a.y, a.z, a.vx, a.vy, a.vz, a.dt, niter,
+                                  correction, rg, &a.memo);
+    if (!hit) return false;
+    a.x += a.vx * a.dt;
+    a.y += a.vy * a.dt;
+    a.z += a.vz * a.dt;
+    a.t += a.dt;
+    if constexpr (kPlain) rg.not_tiny(a.x, a.y);
+    return true;
+}
+
+// The normal at the intersection, reusing Newton's when it was evaluated at
+// this very point.
+template <int K, bool kPlain>
+BT_DEV void arrival_normal(SurfPtr surf, const Arrival& a, double& nx, double& ny,
+                           double& nz, Range& rg)
+{
+    if (a.memo.ok && same_bits(a.memo.dt, a.dt)) {
+        nx = a.memo.nx; ny = a.memo.ny; nz = a.memo.nz;
+    } else {
+        double sag;
+        surf_point<K, kPlain, false, true>(surf, a.x, a.y, sag, nx, ny, nz, rg);
+    }
+}
+
+// One interaction in the plain or the full form, on a ray that has not
+// failed; returns true when the ray's kinematic state was (re)written.
+template <int K, bool kPlain, class Frame>
+BT_DEV bool interact(int action, Frame dr, Frame drot, SurfPtr surf, double n2,
+                     Ray& r, int niter, int start, double correction, Range& rg)
+{
+    Arrival a;
+    if (!arrive<K, kPlain>(dr, drot, surf, r, niter, start, correction, a, rg)) {
+        r.fail = true;
+        r.vig = true;
+        return false;          // left in the previous frame
+    }
+    double nx, ny, nz;
+    if (action == BT_ACT_REFLECT) {                  // batoid.cpp:340-353
+        arrival_normal<K, kPlain>(surf, a, nx, ny, nz, rg);
+        double alpha = a.vx*nx;
+        alpha += a.vy*ny;
+        alpha += a.vz*nz;
+        a.vx -= 2*alpha*nx;
+        a.vy -= 2*alpha*ny;
+        a.vz -= 2*alpha*nz;
+    } else if (action == BT_ACT_REFRACT) {           // batoid.cpp:453-496
+        arrival_normal<K, kPlain>(surf, a, nx, ny, nz, rg);
+        const Incidence c = incidence<kPlain>(nx, ny, nz, a.vx, a.vy, a.vz, rg);
+        if (refract_velocity<kPlain>(c, n2, a.vx, a.vy, a.vz, rg)) {
+            r.fail = true;                           // total internal reflection
+            r.vig = true;
+        }
+    }
+    r.x = a.x; r.y = a.y; r.z = a.z;
+    r.vx = a.vx; r.vy = a.vy; r.vz = a.vz;
+    r.t = a.t;
+    return true;
+}
+
+// A ray that has not failed split at a surface (batoid.cpp:582-672): `r`
+// becomes the refracted part, `q` the reflected one; false where the ray
+// misses, with both parts failed and left in the previous frame.
+template <int K, bool kPlain, class Frame>
+BT_DEV bool split_parts(Frame dr, Frame drot,
+                        SurfPtr surf, double n2, Ray& r, Ray& q, int niter, Range& rg)
+{
+    Arrival a;
+    if (!arrive<K, kPlain>(dr, drot, surf, r, niter, BT_START_REFERENCE, 0.0, a, rg)) {
+        r.fail = true;
+        r.vig = true;
+        q = r;
+        return false;
+    }
+    double nx, ny, nz;
+    arrival_normal<K, kPlain>(surf, a, nx, ny, nz, rg);
+    const Incidence c = incidence<kPlain>(nx, ny, nz, a.vx, a.vy, a.vz, rg);
+    r.x = a.x; r.y = a.y; r.z = a.z;
+    r.t = a.t;
+    q = r;
+    q.vx = a.vx; q.vy = a.vy; q.vz = a.vz;
+    split_reflect<kPlain>(c, q.vx, q.vy, q.vz, rg);
+    if (refract_velocity<kPlain>(c, n2, r.vx, r.vy, r.vz, rg)) {
+        r.fail = true;
+        r.vig = true;
+    }
+    return true;
+}
+
+// split_parts with the wave's vote.
+template <int K, class Frame>
+BT_DEV bool split_ray(Frame dr, Frame drot,
+                      SurfPtr surf, double n2, Ray& r, Ray& q, int niter)
+{
+    Range rg;
+    if constexpr (!kVoted<K>)
+        return split_parts<K, false>(dr, drot, surf, n2, r, q, niter, rg);
+    Ray p = r;
+    bool hit = split_parts<K, true>(dr, drot, surf, n2, p, q, niter, rg);
+    rg.not_tiny(p.vx, p.vy);
+    rg.not_tiny(p.vz, q.vz);
+    rg.not_tiny(q.vx, q.vy);
+    if (__all(rg.plain()))
+        r = p;
+    else
+        hit = split_parts<K, false>(dr, drot, surf, n2, r, q, niter, rg);
+    return hit;
+}
+
 // Returns true when the ray's kinematic state was (re)written.  `n2` is the
 // outgoing medium's index at the ray's wavelength (used by REFRACT only); the
 // reference evaluates it after the intersection (batoid.cpp:474), but it is
 // a pure function of the wavelength, so callers may evaluate it once per ray
 // and medium and reuse it across Interfaces.
-template <int K = kKindsAll>
-BT_DEV bool apply_interaction(int action, const double* __restrict__ dr,
-                              const double* __restrict__ drot,
-                              const bt_surface* surf, double n2,
+template <int K, class Frame>
+BT_DEV bool apply_interaction(int action, Frame dr, Frame drot,
+                              SurfPtr surf, double n2,
                               Ray& r, int niter, int start = BT_START_REFERENCE,
                               double correction = 0.0)
 {
     if (r.fail) return false;
-    double dx = r.x-dr[0];
-    double dy = r.y-dr[1];
-    double dz = r.z-dr[2];
-    double x = dx*drot[0] + dy*drot[3] + dz*drot[6];
-    double y = dx*drot[1] + dy*drot[4] + dz*drot[7];
-    double z = dx*drot[2] + dy*drot[5] + dz*drot[8];
-    double vx = r.vx*drot[0] + r.vy*drot[3] + r.vz*drot[6];
-    double vy = r.vx*drot[1] + r.vy*drot[4] + r.vz*drot[7];
-    double vz = r.vx*drot[2] + r.vy*drot[5] + r.vz*drot[8];
-    double t = r.t;
-    double dt = 0.0;
-    NormalMemo memo;
-    memo.ok = false;
-    const bool hit = (start == BT_START_REFERENCE)
-                         ? surf_tti<K>(surf, x, y, z, vx, vy, vz, dt, niter, &memo)
-                         : fast_tti<K>(surf, x, y, z, vx, vy, vz, dt, niter, correction, &memo);
-    // the normal at the intersection, reusing Newton's when it was evaluated
-    // at this very point
-    auto normal_at = [&](double px, double py, double& nx, double& ny, double& nz) {
-        if (memo.ok && same_bits(memo.dt, dt)) {
-            nx = memo.nx; ny = memo.ny; nz = memo.nz;
-        } else {
-            surf_normal<K>(surf, px, py, nx, ny, nz);
-        }
-    };
-    if (!hit) {
-        r.fail = true;
-        r.vig = true;
-        return false;          // left in the previous frame
-    }
-    x += vx * dt;
-    y += vy * dt;
-    z += vz * dt;
-    t += dt;
-    if (action == BT_ACT_REFLECT) {                  // batoid.cpp:340-353
-        double nx, ny, nz;
-        normal_at(x, y, nx, ny, nz);
-        double alpha = vx*nx;
-        alpha += vy*ny;
-        alpha += vz*nz;
-        vx -= 2*alpha*nx;
-        vy -= 2*alpha*ny;
-        vz -= 2*alpha*nz;
-    } else if (action == BT_ACT_REFRACT) {           // batoid.cpp:453-496
-        double n1 = vx*vx;
-        n1 += vy*vy;
-        n1 += vz*vz;
-        n1 = cr_rsqrt(n1);
-        double nvx = vx*n1;
-        double nvy = vy*n1;
-        double nvz = vz*n1;
-        double nx, ny, nz;
-        normal_at(x, y, nx, ny, nz);
-        double alpha = nvx*nx;
-        alpha += nvy*ny;
-        alpha += nvz*nz;
-        if (alpha > 0.) {
-            nx *= -1; ny *= -1; nz *= -1;
-            alpha *= -1;
-        }
-        // Into a medium of index exactly 1 (vacuum, or air given as a
-        // constant 1) the reference's divisions by n2 return their numerators
-        // bit for bit (x/1 == x in IEEE arithmetic, signed zeros, infinities
-        // and NaNs included), so that case runs without them.
-        auto finish = [&](auto unit) {
-            constexpr bool kUnit = decltype(unit)::value;
-            double eta = n1;
-            if constexpr (!kUnit) eta /= n2;
-            double sinsqr = eta*eta*(1-alpha*alpha);
-            if (sinsqr > 1.0) {                      // total internal reflection
-                vx = __builtin_nan(""); vy = vx; vz = vx;
-                r.fail = true;
-                r.vig = true;
-            } else {
-                double nfactor = eta*alpha + cr_sqrt(1-sinsqr);
-                vx = eta*nvx - nfactor*nx;
-                vy = eta*nvy - nfactor*ny;
-                vz = eta*nvz - nfactor*nz;
-                if constexpr (!kUnit) {
-                    vx /= n2;
-                    vy /= n2;
-                    vz /= n2;
-                }
-            }
-        };
-        if (n2 == 1.0)
-            finish(std::true_type{});
-        else
-            finish(std::false_type{});
-    }
-    r.x = x; r.y = y; r.z = z;
-    r.vx = vx; r.vy = vy; r.vz = vz;
-    r.t = t;
-    return true;
+    Range rg;
+    if constexpr (!kVoted<K>)
+        return interact<K, false>(action, dr, drot, surf, n2, r, niter, start, correction, rg);
+    Ray p = r;
+    bool moved = interact<K, true>(action, dr, drot, surf, n2, p, niter, start, correction, rg);
+    rg.not_tiny(p.vx, p.vy);
+    rg.not_tiny(p.vz, p.vz);
+    if (__all(rg.plain()))
+        r = p;
+    else
+        moved = interact<K, false>(action, dr, drot, surf, n2, r, niter, start, correction, rg);
+    return moved;
 }
 
 }  // namespace bt

@@ -229,8 +229,9 @@ __global__ __launch_bounds__(kBlock) void k_newton_samples(Xform xf, const bt_su
     uint8_t st = 0;
     double dtc = 0.0, dte = 0.0;
     if (!rv.failed[i]) {
-        if (conic_start(surf, x, y, z, vx, vy, vz, dtc)) st |= 1;
-        if (surf_tti(surf, x, y, z, vx, vy, vz, dte, niter)) st |= 2;
+        Range rg;
+        if (conic_start<kKindsAll, false>((SurfPtr)surf, x, y, z, vx, vy, vz, dtc, rg)) st |= 1;
+        if (surf_tti<kKindsAll, false>((SurfPtr)surf, x, y, z, vx, vy, vz, dte, niter, rg)) st |= 2;
     }
     float* f = o.feat + i * kMlpIn;
     f[0] = (float)(x + vx*dtc);

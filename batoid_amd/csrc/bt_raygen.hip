@@ -187,7 +187,7 @@ __global__ __launch_bounds__(kBlock) void k_generate(GenArgs a, bt_rays out)
     default:
         return;   // rejected on the host
     }
-    const double zs = surf_sag(g.stop, xs, ys);
+    const double zs = surf_sag((SurfPtr)g.stop, xs, ys);
     // stop frame -> ray frame (batoid.cpp:8-22)
     const double* dr = g.stop_dr;
     const double* m = g.stop_drot;

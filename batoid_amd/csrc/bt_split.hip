@@ -37,126 +37,55 @@ __device__ __forceinline__ void rsplit_ray(
         if (sp.vignetted) sp.vignetted[i] = 1;
         return;
     }
-    const double* dr = xf.dr;
-    const double* drot = xf.drot;
-    const double x0 = rv.x[i], y0 = rv.y[i], z0 = rv.z[i];
-    const double vx0 = rv.vx[i], vy0 = rv.vy[i], vz0 = rv.vz[i];
-    const double t0 = rv.t[i], w = rv.wavelength[i], f = rv.flux[i];
-    const bool vig0 = rv.vignetted[i] != 0, fail0 = rv.failed[i] != 0;
-    // the split ray starts as a copy of the input (trace.py:125)
-    double sx = x0, sy = y0, sz = z0, svx = vx0, svy = vy0, svz = vz0, st = t0, sf = f;
-    bool svig = vig0, sfail = fail0;
-    // the refracted ray's final position, flag and flux, for the obscuration
-    // and the filter
-    double rx = x0, ry = y0, rf = f;
-    bool rvig = vig0;
+    Ray r;
+    r.x = rv.x[i]; r.y = rv.y[i]; r.z = rv.z[i];
+    r.vx = rv.vx[i]; r.vy = rv.vy[i]; r.vz = rv.vz[i];
+    r.t = rv.t[i];
+    const double w = rv.wavelength[i], f = rv.flux[i];
+    r.vig = rv.vignetted[i] != 0;
+    r.fail = rv.failed[i] != 0;
+    const bool fail0 = r.fail;
+    Ray q = r;                       // the split ray starts as a copy (trace.py:125)
+    double rf = f, sf = f;
+    bool hit = false;
     if (!fail0) {
-        double dx = x0-dr[0];
-        double dy = y0-dr[1];
-        double dz = z0-dr[2];
-        double x = dx*drot[0] + dy*drot[3] + dz*drot[6];
-        double y = dx*drot[1] + dy*drot[4] + dz*drot[7];
-        double z = dx*drot[2] + dy*drot[5] + dz*drot[8];
-        double vx = vx0*drot[0] + vy0*drot[3] + vz0*drot[6];
-        double vy = vx0*drot[1] + vy0*drot[4] + vz0*drot[7];
-        double vz = vx0*drot[2] + vy0*drot[5] + vz0*drot[8];
-        double t = t0;
-        double dt = 0.0;
-        NormalMemo memo;
-        memo.ok = false;
-        const bool hit = surf_tti<K>(surf, x, y, z, vx, vy, vz, dt, niter, &memo);
+        hit = split_ray<K>(xf.dr, xf.drot, (SurfPtr)surf, medium_n((MediumPtr)m2, w), r, q, niter);
         if (hit) {
-            x += vx * dt;
-            y += vy * dt;
-            z += vz * dt;
-            t += dt;
-            double n1 = vx*vx;
-            n1 += vy*vy;
-            n1 += vz*vz;
-            n1 = cr_rsqrt(n1);
-            double nvx = vx*n1;
-            double nvy = vy*n1;
-            double nvz = vz*n1;
-            double nx, ny, nz;
-            if (memo.ok && same_bits(memo.dt, dt)) {  // Newton's last normal, same point
-                nx = memo.nx; ny = memo.ny; nz = memo.nz;
-            } else {
-                surf_normal<K>(surf, x, y, nx, ny, nz);
-            }
-            double alpha = nvx*nx;
-            alpha += nvy*ny;
-            alpha += nvz*nz;
-            if (alpha > 0) {
-                nx *= -1;
-                ny *= -1;
-                nz *= -1;
-                alpha *= -1;
-            }
-            // reflection
-            sx = x; sy = y; sz = z;
-            svx = vx - 2*alpha*nx/n1;
-            svy = vy - 2*alpha*ny/n1;
-            svz = vz - 2*alpha*nz/n1;
-            st = t;
-            sf = f*reflect;
-            // refraction
-            const double n2 = medium_n(m2, w);
-            const double eta = n1/n2;
-            const double sinsqr = eta*eta*(1-alpha*alpha);
-            rv.x[i] = x;
-            rv.y[i] = y;
-            rv.z[i] = z;
-            rv.t[i] = t;
-            rx = x;
-            ry = y;
-            if (sinsqr > 1.0) {                      // total internal reflection
-                const double nan = __builtin_nan("");
-                rv.vx[i] = nan; rv.vy[i] = nan; rv.vz[i] = nan;
-                rv.failed[i] = 1;
-                rv.vignetted[i] = 1;
-                rvig = true;
-            } else {
-                const double nfactor = eta*alpha + cr_sqrt(1-sinsqr);
-                double ux = eta*nvx - nfactor*nx;
-                double uy = eta*nvy - nfactor*ny;
-                double uz = eta*nvz - nfactor*nz;
-                rv.vx[i] = ux / n2;
-                rv.vy[i] = uy / n2;
-                rv.vz[i] = uz / n2;
-            }
             rf = f*transmit;
+            sf = f*reflect;
+            rv.x[i] = r.x; rv.y[i] = r.y; rv.z[i] = r.z;
+            rv.vx[i] = r.vx; rv.vy[i] = r.vy; rv.vz[i] = r.vz;
+            rv.t[i] = r.t;
             rv.flux[i] = rf;
-        } else {
+        }
+        if (r.fail) {
             rv.failed[i] = 1;
             rv.vignetted[i] = 1;
-            rvig = true;
-            svig = true;
-            sfail = true;
         }
     }
     // the Interface's obscuration on both parts (optic.py:491-494), every
     // ray included, as batoid.cpp:151-172
     if (olen > 0) {
-        if (!rvig && obsc_contains(obsc, olen, rx, ry)) {
+        if (!r.vig && obsc_contains((ObscPtr)obsc, olen, r.x, r.y)) {
             rv.vignetted[i] = 1;
-            rvig = true;
+            r.vig = true;
         }
-        if (!svig) svig = obsc_contains(obsc, olen, sx, sy);
+        if (!q.vig) q.vig = obsc_contains((ObscPtr)obsc, olen, q.x, q.y);
     }
-    lr = !rvig && rf >= min_flux;
-    ls = !svig && sf >= min_flux;
+    lr = !r.vig && rf >= min_flux;
+    ls = !q.vig && sf >= min_flux;
     if (!sp.flux) return;                           // no split part asked for
     sp.flux[i] = sf;
-    sp.vignetted[i] = svig;
-    sp.failed[i] = sfail;
+    sp.vignetted[i] = q.vig;
+    sp.failed[i] = q.fail;
     // live mode: a split ray the filter drops (vignetted, or its flux below
     // min_flux -- every one once the ray's flux times the reflectivity is)
     // is never copied out or traced further, and every later pass reads
     // only its flux and flags
     if (live && !ls) return;
-    sp.x[i] = sx; sp.y[i] = sy; sp.z[i] = sz;
-    sp.vx[i] = svx; sp.vy[i] = svy; sp.vz[i] = svz;
-    sp.t[i] = st;
+    sp.x[i] = q.x; sp.y[i] = q.y; sp.z[i] = q.z;
+    sp.vx[i] = q.vx; sp.vy[i] = q.vy; sp.vz[i] = q.vz;
+    sp.t[i] = q.t;
     sp.wavelength[i] = w;
 }
 

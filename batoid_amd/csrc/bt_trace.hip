@@ -10,7 +10,7 @@
 //   * per-surface kernels (bt_intersect/bt_reflect/bt_refract), one HBM read
 //     + write of the touched columns per Interface, with the Interface's
 //     obscuration folded into the same pass;
-//   * the fused plan kernel (bt_trace_plan), which applies every Interface of
+//   * the fused plan kernel (bt_trace_plan, bt_plan.h), which applies every Interface of
 //     an optic while the ray sits in registers: one read and one write per
 //     ray for the whole optic.
 #include <hip/hip_runtime.h>
@@ -23,6 +23,11 @@
 #include "bt_common.h"
 
 namespace bt {
+
+// bt_plan_*.hip
+using PlanLaunch = void(int mode, dim3 grid, hipStream_t st, const bt_plan& plan,
+                        const bt_rays& in, const bt_rays& out, int niter, int need_w);
+PlanLaunch launch_plan_analytic, launch_plan_sum_apb, launch_plan_flat_sums, launch_plan_all;
 
 thread_local std::string g_last_error;
 
@@ -162,9 +167,9 @@ __device__ __forceinline__ bool step_ray(
     double n2 = 0.0;
     if (action == BT_ACT_REFRACT && !r.fail) {
         r.w = rv.wavelength[i];
-        n2 = medium_n(m2, r.w);
+        n2 = medium_n((MediumPtr)m2, r.w);
     }
-    const bool moved = apply_interaction<K>(action, xf.dr, xf.drot, surf, n2, r, niter);
+    const bool moved = apply_interaction<K>(action, xf.dr, xf.drot, (SurfPtr)surf, n2, r, niter);
     if (moved) {
         rv.x[i] = r.x; rv.y[i] = r.y; rv.z[i] = r.z;
         rv.vx[i] = r.vx; rv.vy[i] = r.vy; rv.vz[i] = r.vz;
@@ -176,7 +181,7 @@ __device__ __forceinline__ bool step_ray(
         }
     }
     if (obsc_len > 0 && !r.vig)                     // batoid.cpp:169-171
-        r.vig = obsc_contains(obsc, obsc_len, r.x, r.y);
+        r.vig = obsc_contains((ObscPtr)obsc, obsc_len, r.x, r.y);
     if (r.vig != vig0) rv.vignetted[i] = r.vig;
     if (r.fail != fail0) rv.failed[i] = r.fail;
     return live && !r.vig && f >= min_flux;
@@ -208,153 +213,7 @@ __global__ __launch_bounds__(kBlock) void k_obscure(
     const int64_t i = ray_index();
     if (i >= rv.n) return;
     if (rv.vignetted[i]) return;
-    if (obsc_contains(obsc, obsc_len, rv.x[i], rv.y[i])) rv.vignetted[i] = 1;
-}
-
-// Every step of a plan applied while the ray stays in registers.  A ray's
-// wavelength never changes, so the index of the plan's (first) dispersive
-// medium is evaluated once per ray up front.
-//
-// Mode 0: reference starts only.  Mode 1: CONIC starts honoured (an MLP step
-// runs as CONIC).  Mode 2: MLP starts too; MLP inference is a wave-wide MFMA
-// product, so in this variant every lane of a wave stays in the step loop
-// (lanes past the end work on a copy of the last ray and store nothing).
-//
-// The network's input at an MLP step: the ray's point on the surface's base
-// conic and its direction, in the step's local frame (the frame change is
-// apply_interaction's).
-template <int K>
-__device__ __forceinline__ void mlp_features(const bt_step* __restrict__ st,
-                                             const bt_surface* surf, const Ray& r,
-                                             const MlpPacked* P, float (&f)[kMlpIn])
-{
-    const double* dr = st->dr;
-    const double* m = st->drot;
-    double dx = r.x-dr[0], dy = r.y-dr[1], dz = r.z-dr[2];
-    double x = dx*m[0] + dy*m[3] + dz*m[6];
-    double y = dx*m[1] + dy*m[4] + dz*m[7];
-    double z = dx*m[2] + dy*m[5] + dz*m[8];
-    double vx = r.vx*m[0] + r.vy*m[3] + r.vz*m[6];
-    double vy = r.vx*m[1] + r.vy*m[4] + r.vz*m[7];
-    double vz = r.vx*m[2] + r.vy*m[5] + r.vz*m[8];
-    double dtc = 0.0;
-    if (r.fail || !conic_start<K>(surf, x, y, z, vx, vy, vz, dtc)) {
-        // keep this lane's share of the wave's evaluation finite
-        for (int k = 0; k < kMlpIn; k++) f[k] = P->norm[k];
-        return;
-    }
-    f[0] = (float)(x + vx*dtc);
-    f[1] = (float)(y + vy*dtc);
-    f[2] = (float)(z + vz*dtc);
-    f[3] = (float)vx;
-    f[4] = (float)vy;
-    f[5] = (float)vz;
-}
-
-// Waves per SIMD: the analytic-kinds kernels of modes 0 and 1 are held to
-// five (93 VGPRs, no spills), so that a few more registers in a later change
-// cannot silently drop them to four; the all-kinds kernel
-// of mode 0 is held to four (some registers spill to scratch; the extra
-// wave hides more FP64 latency: 8 % faster on the TMA, 9-12 % on the
-// Newton-heavy optics), mode 2 to three (left alone the compiler would
-// settle for two); the all-kinds kernel of mode 1 keeps the compiler's
-// three, where four measured slower on the TMA.
-// Networks a plan kernel keeps in LDS (45 KB per workgroup).
-constexpr int kMlpLds = 4;
-
-template <int Mode, int K>
-constexpr int plan_waves_per_simd()
-{
-    if (K == kKindsAnalytic && Mode < 2) return 5;
-    if (K == kKindsSumAPB) return Mode == 2 ? 3 : 4;
-    return Mode == 0 ? 4 : (Mode == 2 ? 3 : 1);     // kKindsAll, kKindsFlatSums
-}
-
-template <int Mode, int K>
-__global__ __launch_bounds__(kBlock)
-__attribute__((amdgpu_waves_per_eu(plan_waves_per_simd<Mode, K>())))
-void k_plan(
-    bt_plan plan, bt_rays in, bt_rays out, int niter, int need_w)
-{
-    constexpr bool Fast = Mode > 0;
-    constexpr bool Mlp = Mode > 1;
-    // Mode 2: the networks of the plan's first kMlpLds MLP steps, copied to
-    // LDS once per workgroup (a wave-wide inference then reads its weight
-    // fragments from LDS, not from L2); later MLP steps run as CONIC.
-    const MlpPacked* nets = nullptr;
-    if constexpr (Mlp) {
-        __shared__ MlpPacked lds_nets[kMlpLds];
-        int slot = 0;
-        for (int k = 0; k < plan.nstep && slot < kMlpLds; k++) {
-            const bt_step* st = plan.steps + k;
-            if (st->start != BT_START_MLP || !st->mlp) continue;
-            const uint4* src = static_cast<const uint4*>(st->mlp);
-            uint4* dst = reinterpret_cast<uint4*>(lds_nets + slot);
-            for (int q = threadIdx.x; q < (int)(sizeof(MlpPacked) / 16); q += kBlock)
-                dst[q] = src[q];
-            slot++;
-        }
-        __syncthreads();
-        nets = lds_nets;
-    }
-    const int64_t i0 = ray_index();
-    if (!Mlp && i0 >= in.n) return;
-    const bool live = i0 < in.n;
-    const int64_t i = live ? i0 : in.n - 1;
-    Ray r;
-    r.fail = in.failed[i] != 0;
-    r.vig = in.vignetted[i] != 0;
-    r.x = in.x[i]; r.y = in.y[i]; r.z = in.z[i];
-    r.vx = in.vx[i]; r.vy = in.vy[i]; r.vz = in.vz[i];
-    r.t = in.t[i];
-    // Refractive indices: a constant medium's is its record's (a scalar
-    // load); the plan's first dispersive medium is evaluated once per ray and
-    // kept; any other dispersive medium is evaluated at its refraction, with
-    // the wavelength read again from memory (it is not held in registers).
-    const int nmed = plan.nmedia;
-    int cm = -1;                               // the cached medium (wave-uniform)
-    for (int m = 0; m < nmed; m++)
-        if (plan.media[m].kind != BT_MED_CONST) { cm = m; break; }
-    double ncm = 0.0;
-    if (need_w && cm >= 0 && !r.fail) ncm = medium_n(plan.media + cm, in.wavelength[i]);
-    const int nstep = plan.nstep;
-    int mslot = 0;                             // next LDS network (wave-uniform)
-    for (int k = 0; k < nstep; k++) {
-        if (!Mlp && r.fail && r.vig) break;    // nothing below can change this ray
-        const bt_step* __restrict__ st = plan.steps + k;
-        const bt_surface* surf = plan.surfaces + st->surface;
-        const int action = st->action;
-        double n2 = 0.0;
-        if (action == BT_ACT_REFRACT && !r.fail) {
-            const int mi = st->medium;
-            const bt_medium* med = plan.media + mi;
-            n2 = (med->kind == BT_MED_CONST) ? med->p[0]           // medium.cpp:30-32
-                 : (mi == cm) ? ncm : medium_n(med, in.wavelength[i]);
-        }
-        double correction = 0.0;
-        int start = Fast ? st->start : BT_START_REFERENCE;
-        if (start == BT_START_MLP && (!Mlp || !st->mlp || mslot >= kMlpLds))
-            start = BT_START_CONIC;
-        if (Mlp && start == BT_START_MLP) {     // uniform: whole wave
-            const MlpPacked* P = nets + mslot;
-            mslot++;
-            float f[kMlpIn];
-            mlp_features<K>(st, surf, r, P, f);
-            correction = (double)mlp_predict_wave(P, f);
-        }
-        apply_interaction<K>(action, st->dr, st->drot, surf, n2, r, niter, start, correction);
-        const int olen = st->obsc_len;
-        if (olen > 0 && !r.vig)
-            r.vig = obsc_contains(plan.obscs + st->obsc, olen, r.x, r.y);
-    }
-    if (Mlp && !live) return;
-    out.x[i] = r.x; out.y[i] = r.y; out.z[i] = r.z;
-    out.vx[i] = r.vx; out.vy[i] = r.vy; out.vz[i] = r.vz;
-    out.t[i] = r.t;
-    out.vignetted[i] = r.vig;
-    out.failed[i] = r.fail;
-    if (out.wavelength != in.wavelength) out.wavelength[i] = in.wavelength[i];
-    if (out.flux != in.flux) out.flux[i] = in.flux[i];
+    if (obsc_contains((ObscPtr)obsc, obsc_len, rv.x[i], rv.y[i])) rv.vignetted[i] = 1;
 }
 
 __global__ __launch_bounds__(kBlock) void k_sag(
@@ -363,7 +222,7 @@ __global__ __launch_bounds__(kBlock) void k_sag(
 {
     const int64_t i = ray_index();
     if (i >= n) return;
-    out[i] = surf_sag(s, x[i], y[i]);
+    out[i] = surf_sag((SurfPtr)s, x[i], y[i]);
 }
 
 __global__ __launch_bounds__(kBlock) void k_normal(
@@ -373,7 +232,7 @@ __global__ __launch_bounds__(kBlock) void k_normal(
     const int64_t i = ray_index();
     if (i >= n) return;
     double nx, ny, nz;
-    surf_normal(s, x[i], y[i], nx, ny, nz);
+    surf_normal((SurfPtr)s, x[i], y[i], nx, ny, nz);
     out[i] = nx; out[i+n] = ny; out[i+2*n] = nz;
 }
 
@@ -383,7 +242,7 @@ __global__ __launch_bounds__(kBlock) void k_get_n(
 {
     const int64_t i = ray_index();
     if (i >= n) return;
-    out[i] = medium_n(m, w[i]);
+    out[i] = medium_n((MediumPtr)m, w[i]);
 }
 
 __global__ __launch_bounds__(kBlock) void k_contains(
@@ -392,7 +251,7 @@ __global__ __launch_bounds__(kBlock) void k_contains(
 {
     const int64_t i = ray_index();
     if (i >= n) return;
-    out[i] = obsc_contains(o, len, x[i], y[i]) ? 1 : 0;
+    out[i] = obsc_contains((ObscPtr)o, len, x[i], y[i]) ? 1 : 0;
 }
 
 __global__ __launch_bounds__(kBlock) void k_check_sqrt(
@@ -669,25 +528,11 @@ int bt_trace_plan(bt_plan plan, bt_rays in, bt_rays out, int niter, void* stream
                       : (plan.flags & BT_PLAN_SUM_APB) ? kKindsSumAPB
                       : (plan.flags & BT_PLAN_FLAT_SUMS) ? kKindsFlatSums : kKindsAll;
     const int mode = (plan.flags & BT_PLAN_MLP_START) ? 2 : (plan.flags & BT_PLAN_FAST_START) ? 1 : 0;
-    const dim3 grid(grid_for(in.n)), block(kBlock);
-    hipStream_t st = as_stream(stream);
-#define BT_PLAN_LAUNCH(M, K) \
-    hipLaunchKernelGGL((k_plan<M, K>), grid, block, 0, st, plan, in, out, niter, need_w)
-    switch (mode * 4 + kinds) {
-    case 0: BT_PLAN_LAUNCH(0, kKindsAll); break;
-    case 1: BT_PLAN_LAUNCH(0, kKindsAnalytic); break;
-    case 2: BT_PLAN_LAUNCH(0, kKindsSumAPB); break;
-    case 3: BT_PLAN_LAUNCH(0, kKindsFlatSums); break;
-    case 4: BT_PLAN_LAUNCH(1, kKindsAll); break;
-    case 5: BT_PLAN_LAUNCH(1, kKindsAnalytic); break;
-    case 6: BT_PLAN_LAUNCH(1, kKindsSumAPB); break;
-    case 7: BT_PLAN_LAUNCH(1, kKindsFlatSums); break;
-    case 8: BT_PLAN_LAUNCH(2, kKindsAll); break;
-    case 9: BT_PLAN_LAUNCH(2, kKindsAnalytic); break;
-    case 10: BT_PLAN_LAUNCH(2, kKindsSumAPB); break;
-    default: BT_PLAN_LAUNCH(2, kKindsFlatSums); break;
-    }
-#undef BT_PLAN_LAUNCH
+    const auto launch = kinds == kKindsAnalytic   ? launch_plan_analytic
+                        : kinds == kKindsSumAPB   ? launch_plan_sum_apb
+                        : kinds == kKindsFlatSums ? launch_plan_flat_sums
+                                                  : launch_plan_all;
+    launch(mode, dim3(grid_for(in.n)), as_stream(stream), plan, in, out, niter, need_w);
     return check_launch("bt_trace_plan");
 }
 

@@ -368,7 +368,8 @@ class Bicubic(Surface):
 
     def _leaf_record(self):
         use_nan = 1 if self.nanpolicy.upper() == 'NAN' else 0
-        return (_rec(_lib.BICUBIC, [self._x0, self._y0, self._dx, self._dy],
+        return (_rec(_lib.BICUBIC, [self._x0, self._y0, self._dx, self._dy,
+                                    _div(1., self._dx), _div(1., self._dy)],
                      n1=len(self._xs), n2=len(self._ys), flags=use_nan),
                 (self._zs, self._dzdxs, self._dzdys, self._d2zdxdys))
 

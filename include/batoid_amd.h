@@ -69,8 +69,10 @@ typedef struct bt_rays {
  *   ASPHERE      p as QUADRIC; n1 = ncoef; a0 = coefs (index 0 <-> r^2),
  *                a1 = dz/dr coefs 2(j+1)*coefs[j]         asphere.cpp:10-85
  *   TILTED       p = {tanx, tany}                         tilted.cpp:14-37
- *   BICUBIC      p = {x0, y0, dx, dy}; n1 = nx, n2 = ny; flags = use_nan;
- *                a0..a3 = z, dzdx, dzdy, d2zdxdy row-major [ny][nx]
+ *   BICUBIC      p = {x0, y0, dx, dy, 1/dx, 1/dy}; n1 = nx, n2 = ny;
+ *                flags = use_nan; the reciprocals are optional (0 where not
+ *                given; a value that is not the correctly rounded reciprocal
+ *                is not used) and change no result; a0..a3 = z, dzdx, dzdy, d2zdxdy row-major [ny][nx]
  *                                                         table.cpp:58-158
  *   POLYNOMIAL   p = {xorigin, yorigin}; n1 = xsize, n2 = ysize;
  *                a0 = coefs[ysize][xsize], a1 = gradx, a2 = grady
