@@ -99,8 +99,22 @@ class BtCoating(ctypes.Structure):
     _fields_ = [("reflectivity", ctypes.c_double), ("transmissivity", ctypes.c_double)]
 
 
+class BtChainStep(ctypes.Structure):
+    _fields_ = [
+        ("action", ctypes.c_int32), ("obsc_len", ctypes.c_int32),
+        ("surface", ctypes.c_void_p), ("medium", ctypes.c_void_p), ("obsc", ctypes.c_void_p),
+        ("transmissivity", ctypes.c_double), ("reflectivity", ctypes.c_double),
+        ("dr", ctypes.c_double * 3), ("drot", ctypes.c_double * 9), ("split", BtRays),
+    ]
+
+
+class BtChain(ctypes.Structure):
+    _fields_ = [("steps", ctypes.c_void_p), ("nstep", ctypes.c_int32),
+                ("flags", ctypes.c_int32), ("rays", BtRays)]
+
+
 STRUCTS = (BtRays, BtSurface, BtMedium, BtObsc, BtStep, BtPlan, BtPsfSegment, BtRaygen,
-           BtCoating)
+           BtCoating, BtChainStep, BtChain)
 
 # enum values (include/batoid_amd.h)
 PLANE, SPHERE, PARABOLOID, QUADRIC, ASPHERE, TILTED, BICUBIC, POLYNOMIAL, SUM = range(9)
@@ -108,6 +122,8 @@ MED_CONST, MED_TABLE, MED_SELLMEIER, MED_SUMITA, MED_AIR = range(5)
 (OB_CIRCLE, OB_ANNULUS, OB_RECTANGLE, OB_RAY, OB_POLYGON, OB_NEGATION,
  OB_UNION, OB_INTERSECTION) = range(8)
 ACT_INTERSECT, ACT_REFLECT, ACT_REFRACT = range(3)
+ACT_SPLIT = 3
+CHAIN_FILTERED, CHAIN_NO_OUTPUT = 1, 2
 START_REFERENCE, START_CONIC, START_MLP = range(3)
 PLAN_NO_REFRACT = 1
 PLAN_FAST_START = 2
@@ -148,6 +164,9 @@ SIGNATURES = {
     "bt_select_workspace_bytes": (_L, [_L]),
     "bt_select_count": (_I, [BtRays, _D, _V, _V, _L, _V]),
     "bt_select_scatter": (_I, [BtRays, _D, BtRays, _V, _L, _V]),
+    "bt_select_count_many": (_I, [_V, _I, _L, _D, _V, _V, _L, _V]),
+    "bt_select_scatter_many": (_I, [_V, _V, _I, _L, _D, _V, _L, _V]),
+    "bt_split_chains": (_I, [_V, _I, _L, _D, _I, _I, _V]),
     "bt_obscure": (_I, [_V, _I, BtRays, _V]),
     "bt_trace_plan": (_I, [BtPlan, BtRays, BtRays, _I, _V]),
     "bt_surface_sag": (_I, [_V, _V, _V, _V, _L, _V]),

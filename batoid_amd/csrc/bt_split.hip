@@ -117,6 +117,145 @@ __global__ __launch_bounds__(kBlock) void k_rsplit(
 }
 
 // ---------------------------------------------------------------------------
+// A ray set carried through consecutive Interfaces in one pass (bt_split_chains)
+//
+// Between two reflections a traceSplit set meets every Interface on its way
+// out.  One launch per Interface reads and writes the whole set each time
+// (132 B a ray and Interface, and a launch); here the ray stays in registers
+// over the chain, each split's reflected part goes to its own buffer as it
+// arises, and a ray that the filter drops is only marked dropped in the
+// buffers that follow.  Bytes: the set once in and once out, each reflected
+// ray that is kept once.  Bound by FP64 issue then, as the plan kernel.
+// traceSplit of 998,388 rays, 44 paths: see batoid_amd/split_chain.py.
+// ---------------------------------------------------------------------------
+using ChainStepPtr = const BT_CONSTANT bt_chain_step*;
+using ChainPtr = const BT_CONSTANT bt_chain*;
+using SetPtr = const BT_CONSTANT bt_rays*;
+
+__device__ __forceinline__ bt_rays read_set(SetPtr p)
+{
+    bt_rays r;
+    r.x = p->x; r.y = p->y; r.z = p->z;
+    r.vx = p->vx; r.vy = p->vy; r.vz = p->vz;
+    r.t = p->t; r.wavelength = p->wavelength; r.flux = p->flux;
+    r.vignetted = p->vignetted; r.failed = p->failed;
+    r.n = p->n;
+    return r;
+}
+
+struct ChainRay {
+    Ray r;
+    double flux;
+    bool drop;                       // by the filter, or never kept
+};
+
+template <int K, bool kPlain>
+__device__ __forceinline__ void chain_ray(ChainStepPtr steps, int nstep, bt_rays in, int64_t i,
+                                          double min_flux, int first_live, int niter,
+                                          ChainRay& c, Range& rg)
+{
+    Ray& r = c.r;
+    r.vig = in.vignetted[i] != 0;
+    c.flux = in.flux[i];
+    c.drop = first_live && (r.vig || !(c.flux >= min_flux));
+    r.fail = false;
+    if (!c.drop) {
+        r.fail = in.failed[i] != 0;
+        r.x = in.x[i]; r.y = in.y[i]; r.z = in.z[i];
+        r.vx = in.vx[i]; r.vy = in.vy[i]; r.vz = in.vz[i];
+        r.t = in.t[i];
+    }
+    MediumPtr cached = nullptr;      // the dispersive medium `index` belongs to
+    double index = 0.0;
+    for (int k = 0; k < nstep; k++) {
+        const ChainStepPtr st = steps + k;
+        const SurfPtr surf = (SurfPtr)st->surface;
+        const MediumPtr m2 = (MediumPtr)st->medium;
+        const int action = st->action, olen = st->obsc_len;
+        const bool dispersive = action == BT_ACT_SPLIT && m2->kind != BT_MED_CONST;
+        const bool fresh = dispersive && m2 != cached;
+        if (dispersive) cached = m2;
+        double* const sflux = st->split.flux;
+        if (!c.drop) {
+            if (action == BT_ACT_SPLIT) {
+                Ray q = r;           // the split ray starts as a copy (trace.py:125)
+                double sf = c.flux;
+                if (fresh) index = medium_n(m2, in.wavelength[i]);
+                if (!r.fail && split_parts<K, kPlain>(st->dr, st->drot, surf,
+                                                      dispersive ? index : m2->p[0], r, q,
+                                                      niter, rg)) {
+                    sf = c.flux*st->reflectivity;
+                    c.flux *= st->transmissivity;
+                }
+                if (olen > 0 && !q.vig) q.vig = obsc_contains((ObscPtr)st->obsc, olen, q.x, q.y);
+                if (sflux) {
+                    sflux[i] = sf;
+                    st->split.vignetted[i] = q.vig;
+                    st->split.failed[i] = q.fail;
+                    if (!q.vig && sf >= min_flux) {  // else no later pass reads it
+                        st->split.x[i] = q.x; st->split.y[i] = q.y; st->split.z[i] = q.z;
+                        st->split.vx[i] = q.vx; st->split.vy[i] = q.vy; st->split.vz[i] = q.vz;
+                        st->split.t[i] = q.t;
+                        st->split.wavelength[i] = in.wavelength[i];
+                        if constexpr (kPlain) {
+                            rg.not_tiny(q.vx, q.vy);
+                            rg.not_tiny(q.vz, q.vz);
+                        }
+                    }
+                }
+            } else if (!r.fail) {
+                interact<K, kPlain>(action, st->dr, st->drot, surf, 0.0, r, niter,
+                                    BT_START_REFERENCE, 0.0, rg);
+            }
+            if (olen > 0 && !r.vig) r.vig = obsc_contains((ObscPtr)st->obsc, olen, r.x, r.y);
+            c.drop = r.vig || !(c.flux >= min_flux);
+        } else if (sflux) {
+            st->split.vignetted[i] = 1;
+        }
+    }
+}
+
+// Chain blockIdx.y over its rays: the sets that one turn back after another
+// leaves independent run in one launch (36 sets of 1e6 rays fill the chip for
+// 4 ms; one by one each ended on a nearly empty last round of waves).
+template <int K>
+__global__ __launch_bounds__(kBlock)
+__attribute__((amdgpu_waves_per_eu(K == kKindsAnalytic ? 6 : 3)))
+void k_split_chains(ChainPtr chains, double min_flux, int niter)
+{
+    const ChainPtr chain = chains + blockIdx.y;
+    const bt_rays rays = read_set(&chain->rays);
+    const ChainStepPtr steps = (ChainStepPtr)chain->steps;
+    const int nstep = chain->nstep, flags = chain->flags;
+    const int first_live = (flags & BT_CHAIN_FILTERED) != 0;
+    int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i >= rays.n) return;
+    ChainRay c;
+    Range rg;
+    if constexpr (kVoted<K>) {
+        chain_ray<K, true>(steps, nstep, rays, i, min_flux, first_live, niter, c, rg);
+        if (!c.drop) {
+            rg.not_tiny(c.r.vx, c.r.vy);
+            rg.not_tiny(c.r.vz, c.r.vz);
+        }
+        if (__builtin_expect(!__all(rg.plain()), 0)) {
+            asm("" : "+v"(i));                  // nothing is kept from the plain pass
+            chain_ray<K, false>(steps, nstep, rays, i, min_flux, first_live, niter, c, rg);
+        }
+    } else {
+        chain_ray<K, false>(steps, nstep, rays, i, min_flux, first_live, niter, c, rg);
+    }
+    if (flags & BT_CHAIN_NO_OUTPUT) return;
+    rays.flux[i] = c.flux;
+    rays.vignetted[i] = c.r.vig;
+    rays.failed[i] = c.r.fail;
+    if (first_live && c.drop) return;           // no later pass reads the rest
+    rays.x[i] = c.r.x; rays.y[i] = c.r.y; rays.z[i] = c.r.z;
+    rays.vx[i] = c.r.vx; rays.vy[i] = c.r.vy; rays.vz[i] = c.r.vz;
+    rays.t[i] = c.r.t;
+}
+
+// ---------------------------------------------------------------------------
 // Order-preserving selection: block b covers rays [256 b, 256 b + 256).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ bool selected(const bt_rays& in, int64_t i, double min_flux)
@@ -141,6 +280,20 @@ __device__ __forceinline__ int block_rank(bool keep, int& total)
     return base + __popcll(m & ((1ull << lane) - 1ull));
 }
 
+// The same over blockIdx.y = 0 .. sets of n rays each, with the per-set
+// workspaces side by side: one launch where traceSplit's leaving sets took
+// one each.
+__global__ __launch_bounds__(kBlock) void k_select_count_many(SetPtr sets, double min_flux,
+                                                              int64_t stride,
+                                                              int64_t* __restrict__ counts)
+{
+    const bt_rays in = read_set(sets + blockIdx.y);
+    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    int total;
+    block_rank(selected(in, i, min_flux), total);
+    if (threadIdx.x == 0) counts[blockIdx.y * stride + blockIdx.x] = total;
+}
+
 __global__ __launch_bounds__(kBlock) void k_select_count(bt_rays in, double min_flux,
                                                          int64_t* __restrict__ counts)
 {
@@ -159,8 +312,12 @@ constexpr int kScanPer = 4;
 __global__ __launch_bounds__(kBlock) void k_select_scan(const int64_t* __restrict__ counts,
                                                         int64_t nblocks,
                                                         int64_t* __restrict__ offsets,
-                                                        int64_t* __restrict__ total)
+                                                        int64_t* __restrict__ total,
+                                                        int64_t stride)
 {
+    counts += blockIdx.x * stride;              // one workgroup per set
+    offsets += blockIdx.x * stride;
+    total += blockIdx.x;
     __shared__ int64_t wave_sum[kBlock / 64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int64_t carry = 0;
@@ -195,9 +352,9 @@ __global__ __launch_bounds__(kBlock) void k_select_scan(const int64_t* __restric
     if (threadIdx.x == 0) *total = carry;
 }
 
-__global__ __launch_bounds__(kBlock) void k_select_scatter(bt_rays in, double min_flux,
-                                                           const int64_t* __restrict__ offsets,
-                                                           bt_rays out)
+__device__ __forceinline__ void scatter_ray(const bt_rays& in, double min_flux,
+                                            const int64_t* __restrict__ offsets,
+                                            const bt_rays& out)
 {
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     const bool keep = selected(in, i, min_flux);
@@ -213,6 +370,21 @@ __global__ __launch_bounds__(kBlock) void k_select_scatter(bt_rays in, double mi
     out.flux[o] = in.flux[i];
     out.vignetted[o] = in.vignetted[i];
     out.failed[o] = in.failed[i];
+}
+
+__global__ __launch_bounds__(kBlock) void k_select_scatter(bt_rays in, double min_flux,
+                                                           const int64_t* __restrict__ offsets,
+                                                           bt_rays out)
+{
+    scatter_ray(in, min_flux, offsets, out);
+}
+
+__global__ __launch_bounds__(kBlock) void k_select_scatter_many(
+    SetPtr sets, double min_flux, const int64_t* __restrict__ offsets, int64_t stride, SetPtr outs)
+{
+    const bt_rays in = read_set(sets + blockIdx.y), out = read_set(outs + blockIdx.y);
+    if (out.n == 0) return;
+    scatter_ray(in, min_flux, offsets + blockIdx.y * stride, out);
 }
 
 int64_t select_blocks(int64_t n) { return (n + kBlock - 1) / kBlock; }
@@ -278,6 +450,22 @@ int bt_rsplit_live(const bt_surface* surface, const double* dr, const double* dr
                          min_flux, kinds, counts, stream, "bt_rsplit_live");
 }
 
+int bt_split_chains(const bt_chain* chains, int nchain, int64_t n, double min_flux, int niter,
+                    int kinds, void* stream)
+{
+    if (nchain < 0 || nchain > 65535 || n < 0 || niter < 0)
+        return fail(BT_E_SIZE, "bt_split_chains: bad count");
+    if (n > (int64_t)0x7fffffff * kBlock) return fail(BT_E_SIZE, "bt_split_chains: too many rays");
+    if (nchain == 0 || n == 0) return 0;
+    if (!chains) return fail(BT_E_NULL, "bt_split_chains: null chains");
+    const auto kernel = (kinds & BT_PLAN_ANALYTIC)    ? k_split_chains<kKindsAnalytic>
+                        : (kinds & BT_PLAN_FLAT_SUMS) ? k_split_chains<kKindsFlatSums>
+                                                      : k_split_chains<kKindsAll>;
+    hipLaunchKernelGGL(kernel, dim3(grid_for(n), (unsigned)nchain), dim3(kBlock), 0,
+                       as_stream(stream), (ChainPtr)chains, min_flux, niter);
+    return check_launch("bt_split_chains");
+}
+
 int64_t bt_select_workspace_bytes(int64_t n)
 {
     if (n < 0) return -1;
@@ -303,7 +491,7 @@ int bt_select_count(bt_rays in, double min_flux, int64_t* count, void* workspace
         if (rc) return rc;
     }
     hipLaunchKernelGGL(k_select_scan, dim3(1), dim3(kBlock), 0, s, (const int64_t*)counts, nb,
-                       offsets, count);
+                       offsets, count, (int64_t)0);
     return check_launch("bt_select_count");
 }
 
@@ -321,6 +509,47 @@ int bt_select_scatter(bt_rays in, double min_flux, bt_rays out, const void* work
     hipLaunchKernelGGL(k_select_scatter, dim3((unsigned)nb), dim3(kBlock), 0,
                        as_stream(stream), in, min_flux, offsets, out);
     return check_launch("bt_select_scatter");
+}
+
+int bt_select_count_many(const bt_rays* in, int nset, int64_t n, double min_flux, int64_t* count,
+                         void* workspace, int64_t workspace_bytes, void* stream)
+{
+    if (nset < 0 || nset > 65535 || n < 0) return fail(BT_E_SIZE, "bt_select_count_many: bad count");
+    if (nset == 0) return 0;
+    if (!in || !count || !workspace) return fail(BT_E_NULL, "bt_select_count_many: null argument");
+    if (workspace_bytes / nset < bt_select_workspace_bytes(n))
+        return fail(BT_E_SIZE, "bt_select_count_many: workspace too small");
+    const int64_t nb = select_blocks(n), stride = 2 * (nb + 1);
+    if (nb > 0x7fffffff) return fail(BT_E_SIZE, "bt_select_count_many: too many rays");
+    int64_t* counts = static_cast<int64_t*>(workspace);
+    hipStream_t s = as_stream(stream);
+    if (nb > 0) {
+        hipLaunchKernelGGL(k_select_count_many, dim3((unsigned)nb, (unsigned)nset), dim3(kBlock),
+                           0, s, (SetPtr)in, min_flux, stride, counts);
+        const int rc = check_launch("bt_select_count_many");
+        if (rc) return rc;
+    }
+    hipLaunchKernelGGL(k_select_scan, dim3((unsigned)nset), dim3(kBlock), 0, s,
+                       (const int64_t*)counts, nb, counts + nb + 1, count, stride);
+    return check_launch("bt_select_count_many");
+}
+
+int bt_select_scatter_many(const bt_rays* in, const bt_rays* out, int nset, int64_t n,
+                           double min_flux, const void* workspace, int64_t workspace_bytes,
+                           void* stream)
+{
+    if (nset < 0 || nset > 65535 || n < 0)
+        return fail(BT_E_SIZE, "bt_select_scatter_many: bad count");
+    const int64_t nb = select_blocks(n), stride = 2 * (nb + 1);
+    if (nset == 0 || nb == 0) return 0;
+    if (!in || !out || !workspace) return fail(BT_E_NULL, "bt_select_scatter_many: null argument");
+    if (workspace_bytes / nset < bt_select_workspace_bytes(n))
+        return fail(BT_E_SIZE, "bt_select_scatter_many: workspace too small");
+    if (nb > 0x7fffffff) return fail(BT_E_SIZE, "bt_select_scatter_many: too many rays");
+    const int64_t* offsets = static_cast<const int64_t*>(workspace) + nb + 1;
+    hipLaunchKernelGGL(k_select_scatter_many, dim3((unsigned)nb, (unsigned)nset), dim3(kBlock),
+                       0, as_stream(stream), (SetPtr)in, min_flux, offsets, stride, (SetPtr)out);
+    return check_launch("bt_select_scatter_many");
 }
 
 }  // extern "C"

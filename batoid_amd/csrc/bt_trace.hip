@@ -311,13 +311,14 @@ const char* bt_last_error(void) { return g_last_error.c_str(); }
 
 int bt_struct_sizes(int64_t* sizes, int n)
 {
-    const int64_t all[9] = {(int64_t)sizeof(bt_rays), (int64_t)sizeof(bt_surface),
+    const int64_t all[11] = {(int64_t)sizeof(bt_rays), (int64_t)sizeof(bt_surface),
                             (int64_t)sizeof(bt_medium), (int64_t)sizeof(bt_obsc),
                             (int64_t)sizeof(bt_step), (int64_t)sizeof(bt_plan),
                             (int64_t)sizeof(bt_psf_segment), (int64_t)sizeof(bt_raygen),
-                            (int64_t)sizeof(bt_coating)};
+                            (int64_t)sizeof(bt_coating), (int64_t)sizeof(bt_chain_step),
+                            (int64_t)sizeof(bt_chain)};
     if (!sizes) return fail(BT_E_NULL, "bt_struct_sizes: null argument");
-    for (int i = 0; i < n && i < 9; i++) sizes[i] = all[i];
+    for (int i = 0; i < n && i < 11; i++) sizes[i] = all[i];
     return 0;
 }
 
@@ -362,24 +363,32 @@ const FieldOffset kRaygenFields[] = {
     BT_F(bt_raygen, flux0)};
 const FieldOffset kCoatingFields[] = {
     BT_F(bt_coating, reflectivity), BT_F(bt_coating, transmissivity)};
+const FieldOffset kChainFields[] = {
+    BT_F(bt_chain, steps), BT_F(bt_chain, nstep), BT_F(bt_chain, flags), BT_F(bt_chain, rays)};
+const FieldOffset kChainStepFields[] = {
+    BT_F(bt_chain_step, action), BT_F(bt_chain_step, obsc_len), BT_F(bt_chain_step, surface),
+    BT_F(bt_chain_step, medium), BT_F(bt_chain_step, obsc), BT_F(bt_chain_step, transmissivity),
+    BT_F(bt_chain_step, reflectivity), BT_F(bt_chain_step, dr), BT_F(bt_chain_step, drot),
+    BT_F(bt_chain_step, split)};
 #undef BT_F
 #define BT_TABLE(t) {t, (int)(sizeof(t) / sizeof(t[0]))}
-const struct { const FieldOffset* fields; int count; } kStructFields[9] = {
+const struct { const FieldOffset* fields; int count; } kStructFields[11] = {
     BT_TABLE(kRaysFields), BT_TABLE(kSurfaceFields), BT_TABLE(kMediumFields),
     BT_TABLE(kObscFields), BT_TABLE(kStepFields), BT_TABLE(kPlanFields),
-    BT_TABLE(kSegmentFields), BT_TABLE(kRaygenFields), BT_TABLE(kCoatingFields)};
+    BT_TABLE(kSegmentFields), BT_TABLE(kRaygenFields), BT_TABLE(kCoatingFields),
+    BT_TABLE(kChainStepFields), BT_TABLE(kChainFields)};
 #undef BT_TABLE
 }  // namespace
 
 int bt_struct_field_count(int which)
 {
-    if (which < 0 || which >= 9) return fail(BT_E_SIZE, "bt_struct_field_count: no such struct");
+    if (which < 0 || which >= 11) return fail(BT_E_SIZE, "bt_struct_field_count: no such struct");
     return kStructFields[which].count;
 }
 
 int64_t bt_struct_field_offset(int which, const char* field)
 {
-    if (which < 0 || which >= 9 || !field) return -1;
+    if (which < 0 || which >= 11 || !field) return -1;
     for (int i = 0; i < kStructFields[which].count; i++)
         if (strcmp(kStructFields[which].fields[i].name, field) == 0)
             return kStructFields[which].fields[i].offset;

@@ -9,7 +9,7 @@ from functools import cached_property
 import numpy as np
 import torch
 
-from . import _lib, _device
+from . import _lib, _device, split_chain
 from .constants import globalCoordSys, vacuum
 from .obscuration import ObscNegation, ObscCircle, ObscAnnulus
 from .coating import SimpleCoating
@@ -624,6 +624,8 @@ class CompoundOptic(Optic):
         bound = None if _verbose else self._flux_bound(rv, minFlux)
         if bound is None:
             return self._split_batch([(rv, reverse, False)], minFlux, _verbose)[0]
+        if split_chain.supported(self) and not self.skip:
+            return split_chain.trace_split(self, rv, reverse, minFlux, bound)
         rv._flux_bound = bound
         try:
             return self._split_batch([(rv, reverse, False)], minFlux, _deferred=True)[0]

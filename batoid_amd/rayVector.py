@@ -627,14 +627,22 @@ class _SelectCounts:
         lib = _lib.load()
         self.rvs = rvs
         self.minFlux = float(minFlux)
+        n = len(rvs[0]) if rvs else 0
+        # sets of one size (traceSplit's leaving sets) take one launch
+        self.many = 1 < len(rvs) <= 65535 and all(len(rv) == n for rv in rvs)
         self.sizes = [int(lib.bt_select_workspace_bytes(len(rv))) for rv in rvs]
         self.offs, tot = [], 0
         for b in self.sizes:
             self.offs.append(tot)
-            tot += -(-b // 256) * 256
+            tot += b if self.many else -(-b // 256) * 256
         self.ws = torch.empty(tot + 8 * len(rvs), dtype=torch.uint8, device=_device.device())
         self.counts = self.ws[tot:].view(torch.int64)   # written by bt_select_count
         stream = _device.stream()
+        if self.many:
+            self.table = _device.upload_bytes(_lib.struct_array_bytes([rv._rays for rv in rvs]))
+            _lib.call("bt_select_count_many", _device.ptr(self.table), len(rvs), n, self.minFlux,
+                      _device.ptr(self.counts), _device.ptr(self.ws), tot, stream)
+            return
         for i, rv in enumerate(rvs):
             _lib.call("bt_select_count", rv._rays, self.minFlux, _device.ptr(self.counts[i:]),
                       _device.ptr(self.ws[self.offs[i]:]), self.sizes[i], stream)
@@ -646,3 +654,14 @@ class _SelectCounts:
             _lib.call("bt_select_scatter", rv._rays, self.minFlux, out._rays,
                       _device.ptr(self.ws[self.offs[i]:]), self.sizes[i], _device.stream())
         return out
+
+    def scatter_all(self, counts):
+        """``[self.scatter(i, m) for i, m in enumerate(counts)]``."""
+        if not self.many:
+            return [self.scatter(i, m) for i, m in enumerate(counts)]
+        outs = [RayVector._empty(m, rv.coordSys) for rv, m in zip(self.rvs, counts)]
+        table = _device.upload_bytes(_lib.struct_array_bytes([o._rays for o in outs]))
+        _lib.call("bt_select_scatter_many", _device.ptr(self.table), _device.ptr(table),
+                  len(outs), len(self.rvs[0]), self.minFlux, _device.ptr(self.ws),
+                  sum(self.sizes), _device.stream())
+        return outs

@@ -72,7 +72,8 @@ typedef struct bt_rays {
  *   BICUBIC      p = {x0, y0, dx, dy, 1/dx, 1/dy}; n1 = nx, n2 = ny;
  *                flags = use_nan; the reciprocals are optional (0 where not
  *                given; a value that is not the correctly rounded reciprocal
- *                is not used) and change no result; a0..a3 = z, dzdx, dzdy, d2zdxdy row-major [ny][nx]
+ *                is not used) and change no result;
+ *                a0..a3 = z, dzdx, dzdy, d2zdxdy row-major [ny][nx]
  *                                                         table.cpp:58-158
  *   POLYNOMIAL   p = {xorigin, yorigin}; n1 = xsize, n2 = ysize;
  *                a0 = coefs[ysize][xsize], a1 = gradx, a2 = grady
@@ -341,6 +342,33 @@ typedef struct bt_coating {
     double transmissivity;
 } bt_coating;
 
+/* ---- split chains -------------------------------------------------------
+ * One Interface of a ray set's way through an optic between two turns back
+ * (bt_split_chains).  SPLIT refracts the rays in place into `medium` and
+ * writes the reflected parts to `split` (every column NULL: not asked for);
+ * REFLECT and INTERSECT are a Mirror's and a Baffle's steps.               */
+#define BT_ACT_SPLIT 3
+typedef struct bt_chain_step {
+    int32_t action;             /* BT_ACT_SPLIT, _REFLECT or _INTERSECT     */
+    int32_t obsc_len;           /* obscuration of both parts, 0 for none    */
+    const bt_surface* surface;  /* records of this step alone               */
+    const bt_medium* medium;    /* outgoing medium of a SPLIT               */
+    const bt_obsc* obsc;
+    double transmissivity, reflectivity;     /* flux factors of a SPLIT     */
+    double dr[3], drot[9];      /* from the previous step's frame           */
+    bt_rays split;
+} bt_chain_step;
+
+/* A ray set and the steps it takes (DEVICE array `steps`).                 */
+#define BT_CHAIN_FILTERED  1    /* the filter already applies to `rays`     */
+#define BT_CHAIN_NO_OUTPUT 2    /* the continuing rays are not written back */
+typedef struct bt_chain {
+    const bt_chain_step* steps;
+    int32_t nstep;
+    int32_t flags;
+    bt_rays rays;
+} bt_chain;
+
 /* ---- per-surface trace --------------------------------------------------
  * Replace _batoid.intersect / reflect / refract (src/batoid.cpp:175-506,
  * pysrc/batoid.cpp:55-57) with the caller's niter.  `surface` is a device
@@ -426,6 +454,31 @@ int bt_select_count(bt_rays in, double min_flux, int64_t* count, void* workspace
                     int64_t workspace_bytes, void* stream);
 int bt_select_scatter(bt_rays in, double min_flux, bt_rays out, const void* workspace,
                       int64_t workspace_bytes, void* stream);
+
+/* The same two calls over `nset` (at most 65535) ray sets of n rays each:
+ * `in` and `out` are DEVICE arrays of nset records, count[nset] as above, an
+ * `out` with n = 0 is not written.  Workspace: nset times
+ * bt_select_workspace_bytes(n).                                            */
+int bt_select_count_many(const bt_rays* in, int nset, int64_t n, double min_flux, int64_t* count,
+                         void* workspace, int64_t workspace_bytes, void* stream);
+int bt_select_scatter_many(const bt_rays* in, const bt_rays* out, int nset, int64_t n,
+                           double min_flux, const void* workspace, int64_t workspace_bytes,
+                           void* stream);
+
+/* traceSplit's steps for ray sets between two turns back, each set in one
+ * pass: `nchain` (at most 65535) records of the DEVICE array `chains`, every
+ * rays.n = n, every column of their rays and of the splits asked for given,
+ * no set twice.  Each step runs as bt_rsplit_live / bt_interact_live would
+ * (same kept rays, bit for bit).  A ray that the filter (bt_select_count's)
+ * has dropped -- before the first step only with BT_CHAIN_FILTERED -- goes no
+ * further: its later reflected parts are marked vignetted and nothing else
+ * of them is written; a reflected part that the filter drops is written as
+ * its flux and flags.  The continuing rays are written back in place, of a
+ * dropped ray of a filtered set the flux and flags only.  `kinds`:
+ * BT_PLAN_ANALYTIC or BT_PLAN_FLAT_SUMS where every step's surface allows,
+ * as for a plan.                                                           */
+int bt_split_chains(const bt_chain* chains, int nchain, int64_t n, double min_flux, int niter,
+                    int kinds, void* stream);
 
 /* Replaces _batoid.obscure (src/batoid.cpp:151-172, pysrc/batoid.cpp:59). */
 int bt_obscure(const bt_obsc* obsc, int obsc_len, bt_rays rays, void* stream);

@@ -1,0 +1,71 @@
+"""bt_split_chains: traceSplit with each set carried through its chain of
+Interfaces in one pass gives the counted rounds' sets, order and bits."""
+import numpy as np
+import pytest
+
+import batoid_amd as bt
+from batoid_amd import workloads
+
+from helpers import assert_cols_identical, FCOLS, BCOLS
+
+pytestmark = pytest.mark.gpu
+
+
+class OwnLens(bt.RefractiveInterface):
+    """A subclass: its rSplit may differ, so chains are not taken."""
+
+
+def coated(optic, r=0.02):
+    for item in optic.itemDict.values():
+        if isinstance(item, bt.RefractiveInterface):
+            item.forwardCoating = item.reverseCoating = bt.SimpleCoating(r, 1 - r)
+        if isinstance(item, bt.Detector):
+            item.forwardCoating = bt.SimpleCoating(r, 1 - r)
+    return optic
+
+
+def optics(name):
+    optic = workloads.perturbed_tma(grid=24) if name in ("perturbed", "nested") else workloads.tma()
+    if name == "nested":
+        m2 = optic['M2'].surface
+        optic = optic.withSurface('M2', bt.Sum(bt.Sum(*m2.surfaces[:2]), m2.surfaces[2]))
+    if name == "baffle":
+        optic = optic.withInsertedOptic('M3', bt.Baffle(
+            bt.Plane(), name='B', coordSys=bt.CoordSys().shiftGlobal([0, 0, 2.0]),
+            obscuration=bt.ObscNegation(bt.ObscCircle(3.0))))
+    if name == "skip":
+        optic['Filter'].skip = True
+    if name == "subclass":
+        optic['L1_entrance'].__class__ = OwnLens
+    return coated(optic)
+
+
+def host(rv):
+    return {k: getattr(rv, k) for k in FCOLS + BCOLS}
+
+
+@pytest.mark.parametrize("name,n,minFlux", [
+    ("tma", 1, 1e-3), ("tma", 255, 1e-4), ("tma", 256, 1e-5), ("tma", 2561, 1e-4),
+    ("baffle", 257, 1e-4), ("skip", 700, 1e-4), ("perturbed", 511, 1e-4), ("nested", 300, 1e-3),
+    ("subclass", 300, 1e-4)])
+def test_chains_equal_counted_rounds(monkeypatch, name, n, minFlux):
+    optic = optics(name)
+    rv = bt.RayVector.asPolar(optic=optic, nrandom=n, rng=np.random.default_rng(n),
+                              wavelength=620e-9, theta_x=0.011, theta_y=-0.007)
+    cols = host(rv)
+    k = np.arange(n)
+    cols["flux"] = np.where(k % 7 == 3, 0.5 * minFlux, np.where(k % 5 == 1, 1.5, 0.8))
+    cols["vignetted"] = k % 11 == 4
+    cols["failed"] = k % 22 == 4                     # vignetted ones only
+    cols["x"][k % 9 == 2] = cols["y"][k % 9 == 2] = 0.0
+    rays = bt.RayVector(**cols, coordSys=rv.coordSys)
+    got = optic.traceSplit(rays.copy(), minFlux=minFlux)
+    with monkeypatch.context() as mp:
+        mp.setattr(bt.CompoundOptic, "_flux_bound", lambda self, rv, m: None)
+        want = optic.traceSplit(rays.copy(), minFlux=minFlux)
+    for g, w in zip(got, want):
+        assert [r.path for r in g] == [r.path for r in w]
+        for a, b in zip(g, w):
+            assert len(a) == len(b) and a.coordSys == b.coordSys
+            assert_cols_identical(host(a), host(b), what=f"{name} {'/'.join(a.path)}")
+    assert n < 200 or sum(map(len, got)) > 3
