@@ -241,21 +241,25 @@ constexpr int gemm_threads() { return gemm_cb<kPrec>() == 4 ? 128 : 256; }
 template <int kPrec>
 constexpr int gemm_waves_per_simd() { return gemm_cb<kPrec>() == 4 ? 1 : 2; }
 
-// One workgroup's 128 x 128 complex tile of the sum over rays [r0, r1) of
-// the prepared parameters, written as FP32 (re, im) into out[i][j][2] (the
-// padded nxp x nyp image).  Every lane of the workgroup must call it.
-template <int kPrec>
+// Wave `wave`'s part of a 128 x 128 complex tile of the sum over rays [r0,
+// r1) of the prepared parameters, written as FP32 (re, im) into out[i][j][2]
+// (the padded nxp x nyp image).  kCols (FP32): 0 for the wave's four column
+// blocks, 1 or 2 for the first or last two of them alone, with the same
+// operands and sums, bit for bit.  Every lane of the wave must call it.
+template <int kPrec, int kCols>
 __device__ __forceinline__ void psf_tile(const float* __restrict__ params,
                                          const float* __restrict__ rot, int r0, int r1,
-                                         int tile_i0, int tile_j0, int nx, int ny, int nyp,
-                                         float* __restrict__ out)
+                                         int tile_i0, int tile_j0, int wave, int nx, int ny,
+                                         int nyp, float* __restrict__ out)
 {
+    static_assert(kCols == 0 || kPrec == BT_PSF_FP32, "split-BF16 takes whole halves");
     // column blocks of 32 per wave: 4 (64 x 128) or 2 (split-BF16 64 x 64)
-    constexpr int CB = gemm_cb<kPrec>();
+    constexpr int CB = kCols == 0 ? gemm_cb<kPrec>() : 2;
+    constexpr int kFirst = kCols == 2 ? 2 : 0;        // first column block taken
     const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
     const int i0 = tile_i0 + (wave & 1) * 64;
-    const int j0 = tile_j0 + (wave >> 1) * (32 * CB);
+    const int jbase = tile_j0 + (wave >> 1) * (32 * gemm_cb<kPrec>());
+    const int j0 = jbase + 32 * kFirst;
     const int half = lane >> 5;       // k half of the operand
     const int l32 = lane & 31;
     v16f acc[4][CB];
@@ -267,7 +271,7 @@ __device__ __forceinline__ void psf_tile(const float* __restrict__ params,
     float ci[4], cj[CB];
     const int prow = l32 & 1;                          // re / im row
     for (int rb = 0; rb < 4; rb++) ci[rb] = (float)(i0 + rb*16 + (l32 >> 1) - nx/2);
-    for (int cb = 0; cb < CB; cb++) cj[cb] = (float)(j0 + cb*32 + l32 - ny/2);
+    for (int cb = 0; cb < CB; cb++) cj[cb] = (float)(jbase + cb*32 + l32 - ny/2);
 
     if constexpr (kPrec == BT_PSF_FP32) {
         // 32x32x2: lane supplies A'[l32][half], B'[half][l32]; one ray per MFMA
@@ -318,10 +322,11 @@ __device__ __forceinline__ void psf_tile(const float* __restrict__ params,
             const float qc[3] = {F(d.e.x), F(d.e.z), F(d.f.x)};
             const float qs[3] = {F(d.e.y), F(d.e.w), F(d.f.y)};
             av[0] = as;
-            bv[0] = bs;
-            for (int k = 1; k < 4; k++) {
+            for (int k = 1; k < 4; k++)
                 av[k] = __builtin_fmaf(as, rc[k - 1], ac * rs[k - 1]);
-                bv[k] = __builtin_fmaf(bs, qc[k - 1], bc * qs[k - 1]);
+            for (int cb = 0; cb < CB; cb++) {
+                const int k = kFirst + cb;
+                bv[cb] = k == 0 ? bs : __builtin_fmaf(bs, qc[k - 1], bc * qs[k - 1]);
             }
         };
         // Software pipeline, one wave per SIMD.  Step r: the MFMAs of ray r
@@ -343,9 +348,9 @@ __device__ __forceinline__ void psf_tile(const float* __restrict__ params,
                 for (int cb = 0; cb < CB; cb++)
                     acc[rb][cb] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[ia][rb], bv[ia][cb],
                                                                       acc[rb][cb], 0, 0, 0);
-            for (int k = 0; k < 2 * CB; k++) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);   // two MFMAs
-                __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);   // four VALU
+            for (int k = 0; k < 8; k++) {
+                __builtin_amdgcn_sched_group_barrier(0x008, CB / 2, 0);   // MFMAs
+                __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);        // four VALU
             }
             __builtin_amdgcn_sched_barrier(0);
         };
@@ -481,7 +486,9 @@ __device__ __forceinline__ void psf_tile(const float* __restrict__ params,
     }
 
     // D[row][col]: row = 8*(e/4) + 4*half + e%4, col = l32 (32x32 MFMA layout)
-    // out[i][j][2] over the padded nxp x nyp image
+    // out[i][j][2] over the padded nxp x nyp image; of a wave's tile that
+    // reaches past the image only the image's part is written (and read)
+    const bool inside = i0 + 64 <= nx && j0 + 32 * CB <= ny;
 #pragma unroll
     for (int rb = 0; rb < 4; rb++)
 #pragma unroll
@@ -491,10 +498,10 @@ __device__ __forceinline__ void psf_tile(const float* __restrict__ params,
                 const int row = 8*(e >> 2) + 4*half + (e & 3);
                 const int i = i0 + rb*16 + (row >> 1);
                 const int j = j0 + cb*32 + l32;
-                out[((int64_t)i * nyp + j) * 2 + (row & 1)] = acc[rb][cb][e];
+                if (inside || (i < nx && j < ny))
+                    out[((int64_t)i * nyp + j) * 2 + (row & 1)] = acc[rb][cb][e];
             }
 }
-
 
 template <int kPrec>
 __global__ __launch_bounds__(gemm_threads<kPrec>(), gemm_waves_per_simd<kPrec>()) void k_psf_gemm(
@@ -509,49 +516,55 @@ __global__ __launch_bounds__(gemm_threads<kPrec>(), gemm_waves_per_simd<kPrec>()
     per = ((per + kRayGroup - 1) / kRayGroup) * kRayGroup;
     const int r0 = ks * per;
     const int r1 = min(total, r0 + per);
-    psf_tile<kPrec>(params, rot, r0, r1, (tile % tiles_i) * kTile, (tile / tiles_i) * kTile, nx, ny,
-                    nyp, partial + (int64_t)ks * nxp * nyp * 2);
+    psf_tile<kPrec, 0>(params, rot, r0, r1, (tile % tiles_i) * kTile, (tile / tiles_i) * kTile,
+                       threadIdx.x >> 6, nx, ny, nyp, partial + (int64_t)ks * nxp * nyp * 2);
 }
 
 // amp[j][i] = sum_ks partial[ks][i][j] in FP64, in a fixed order: a block
-// covers 32 consecutive pixels (j fastest, coalesced float2 reads) with 8
-// lanes per pixel, lane g summing splits g, g+8, ...; the 8 sums are then
-// added in g order.
+// covers kRedPix consecutive pixels (j fastest, coalesced float2 reads) with
+// L lanes per pixel, lane g summing splits g, g+L, ...; the L sums are then
+// added in g order.  Bound by the partial images' reads once enough of them
+// are in flight: 8 lanes read the 128 splits of a 256 x 256 image at 6.3
+// TB/s, but the 512 splits of a 75 x 75 one (176 blocks) at 1.1 TB/s; 32
+// lanes take those from 21.6 to 7 us.
 constexpr int kRedPix = 32;
-constexpr int kRedLanes = kBlock / kRedPix;
 
+template <int L>
 __device__ __forceinline__ void reduce_splits(const float2* __restrict__ p, int64_t stride,
                                               int k0, int k1, bool live, double* __restrict__ out)
 {
-    __shared__ double s_re[kRedLanes][kRedPix], s_im[kRedLanes][kRedPix];
+    __shared__ double s_re[L][kRedPix], s_im[L][kRedPix];
     const int pj = threadIdx.x % kRedPix, g = threadIdx.x / kRedPix;
     double re = 0.0, im = 0.0;
-    if (live)
-        for (int k = k0 + g; k < k1; k += kRedLanes) {
+    if (live) {
+#pragma unroll 4
+        for (int k = k0 + g; k < k1; k += L) {
             const float2 v = p[k * stride];
             re += (double)v.x;
             im += (double)v.y;
         }
+    }
     s_re[g][pj] = re;
     s_im[g][pj] = im;
     __syncthreads();
     if (g == 0 && live) {
         double r = 0.0, m = 0.0;
-        for (int q = 0; q < kRedLanes; q++) { r += s_re[q][pj]; m += s_im[q][pj]; }
+        for (int q = 0; q < L; q++) { r += s_re[q][pj]; m += s_im[q][pj]; }
         out[0] = r;
         out[1] = m;
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_psf_reduce(const float* __restrict__ partial,
-                                                       int ksplit, int nx, int ny, int nxp,
-                                                       int nyp, double* __restrict__ amp)
+template <int L>
+__global__ __launch_bounds__(L * kRedPix) void k_psf_reduce(const float* __restrict__ partial,
+                                                            int ksplit, int nx, int ny, int nxp,
+                                                            int nyp, double* __restrict__ amp)
 {
     const int64_t q = (int64_t)blockIdx.x * kRedPix + threadIdx.x % kRedPix;
     const bool live = q < (int64_t)nx * ny;
     const int i = live ? (int)(q / ny) : 0, j = live ? (int)(q % ny) : 0;
     const float2* p = reinterpret_cast<const float2*>(partial) + ((int64_t)i * nyp + j);
-    reduce_splits(p, (int64_t)nxp * nyp, 0, ksplit, live, amp + 2 * ((int64_t)j * nx + i));
+    reduce_splits<L>(p, (int64_t)nxp * nyp, 0, ksplit, live, amp + 2 * ((int64_t)j * nx + i));
 }
 
 // ---------------------------------------------------------------------------
@@ -650,13 +663,17 @@ __global__ __launch_bounds__(kBlock) void k_psf_prep_batch(
              orot);
 }
 
-// Number of valid rays before ray index b (b <= n), from the block offsets.
+// Number of valid rays before ray index b (b <= n), from the block offsets,
+// by one wave.
 __device__ __forceinline__ int valid_before(const bt_rays& rv, const int* __restrict__ offsets,
                                             int64_t b, int ignore_vig)
 {
     const int64_t blk = b / kBlock;
     int c = offsets[blk];
-    for (int64_t i = blk * kBlock; i < b; i++) c += psf_valid(rv, i, ignore_vig) ? 1 : 0;
+    for (int64_t i0 = blk * kBlock; i0 < b; i0 += 64) {
+        const int64_t i = i0 + (threadIdx.x & 63);
+        c += __popcll(__ballot(i < b && psf_valid(rv, i, ignore_vig)));
+    }
     return c;
 }
 
@@ -667,11 +684,13 @@ struct SegRange {
     int first;      // index of the segment's first work item
 };
 
+// One wave per segment (a thread per segment walked up to 255 flags of a
+// block one by one: 98 us for 96 segments, against 4).
 __global__ __launch_bounds__(kBlock) void k_psf_seg_ranges(
     bt_rays rv, const bt_psf_segment* __restrict__ segs, int nseg, int ignore_vig,
     const int* __restrict__ offsets, int chunk, SegRange* __restrict__ ranges)
 {
-    const int sg = blockIdx.x * kBlock + threadIdx.x;
+    const int sg = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
     if (sg >= nseg) return;
     const bt_psf_segment d = segs[sg];
     const int64_t b = d.begin < 0 ? 0 : (d.begin > rv.n ? rv.n : d.begin);
@@ -683,27 +702,39 @@ __global__ __launch_bounds__(kBlock) void k_psf_seg_ranges(
     r.count = ce - cb;
     r.items = (r.count + chunk - 1) / chunk;
     r.first = 0;
-    ranges[sg] = r;
+    if ((threadIdx.x & 63) == 0) ranges[sg] = r;
 }
 
 struct WorkItem {
-    int seg, r0, r1, pad;
+    int seg, r0, r1;
+    int place;      // its partial image: the segment's first + its number there
 };
 
-// Exclusive scan of the segments' item counts, then the item list
-// (segment-major, chunks in ray order); items[cap..] are never written and
-// *nitems is clamped to cap.
+// The items (chunks of `chunk` rays of each segment and its remainder) by an
+// exclusive scan of the segments' counts, listed by falling length in
+// kItemClasses classes (a counting sort; the order inside a class is free, a
+// partial image's place is not: its segment's, in ray order).  items[cap..]
+// are never written and *nitems is clamped to cap.  *queue is cleared for the
+// GEMM launch.
+constexpr int kItemClasses = 32;
+
 __global__ __launch_bounds__(kScanThreads) void k_psf_items(SegRange* __restrict__ ranges,
                                                             int nseg, int chunk, int cap,
                                                             WorkItem* __restrict__ items,
-                                                            int* __restrict__ nitems)
+                                                            int* __restrict__ nitems,
+                                                            unsigned long long* __restrict__ queue)
 {
     __shared__ int s[kScanThreads];
+    __shared__ int place[kItemClasses];
     const int per = (nseg + kScanThreads - 1) / kScanThreads;
     const int s0 = threadIdx.x * per;
+    auto cls = [&](int len) {                    // 0: the longest
+        return (int)((int64_t)(chunk - len) * kItemClasses / (chunk + 1));
+    };
     int sum = 0;
     for (int q = s0; q < s0 + per && q < nseg; q++) sum += ranges[q].items;
     s[threadIdx.x] = sum;
+    if (threadIdx.x < kItemClasses) place[threadIdx.x] = 0;
     __syncthreads();
     for (int d = 1; d < kScanThreads; d <<= 1) {
         int v = (threadIdx.x >= d) ? s[threadIdx.x - d] : 0;
@@ -711,62 +742,122 @@ __global__ __launch_bounds__(kScanThreads) void k_psf_items(SegRange* __restrict
         s[threadIdx.x] += v;
         __syncthreads();
     }
+    const int total = min(s[kScanThreads - 1], cap);
     int run = s[threadIdx.x] - sum;
     for (int q = s0; q < s0 + per && q < nseg; q++) {
         SegRange r = ranges[q];
         r.first = run;
         ranges[q] = r;
-        for (int c = 0; c < r.items; c++) {
-            const int it = run + c;
-            if (it >= cap) break;
-            const int r0 = r.begin + c * chunk;
-            const int r1 = min(r.begin + r.count, r0 + chunk);
-            items[it] = WorkItem{q, r0, r1, 0};
-        }
+        const int whole = max(0, min(r.count / chunk, cap - run));
+        if (whole > 0) atomicAdd(&place[0], whole);
+        if (r.items > whole && run + whole < cap)
+            atomicAdd(&place[cls(r.count - whole * chunk)], 1);
         run += r.items;
     }
-    if (threadIdx.x == kScanThreads - 1) {
-        const int total = s[kScanThreads - 1];
-        *nitems = total < cap ? total : cap;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int at = 0;
+        for (int k = 0; k < kItemClasses; k++) {
+            const int c = place[k];
+            place[k] = at;
+            at += c;
+        }
+        *nitems = total;
+        *queue = 0;
+    }
+    __syncthreads();
+    for (int q = s0; q < s0 + per && q < nseg; q++) {
+        const SegRange r = ranges[q];
+        for (int c = 0; c < r.items && r.first + c < cap; c++) {
+            const int r0 = r.begin + c * chunk;
+            const int r1 = min(r.begin + r.count, r0 + chunk);
+            const int at = atomicAdd(&place[cls(r1 - r0)], 1);
+            items[at] = WorkItem{q, r0, r1, r.first + c};
+        }
     }
 }
 
-// Persistent GEMM: workgroup w takes (item, tile) pairs w, w + grid, ... in a
-// fixed assignment, so the result does not depend on scheduling.
+// Persistent GEMM over a queue of units, one wave each at a time (the FP32
+// wave's accumulators fill a SIMD's registers): a unit is an item and one of
+// the 64 x 128 halves of a tile, or, where those would leave SIMDs idle
+// (fewer than two a SIMD), one of its 64 x 64 quarters, FP32 only.  A unit's
+// sums do not depend on which wave takes it or when, and a quarter's are the
+// half's bit for bit, so results do not depend on scheduling.  96 segments of
+// ~5,100 rays (288 items of 2,048 rays or less, 128 x 128 pixels): 0.78 ms,
+// 1.10 with a fixed assignment of items to two-wave workgroups, which left 448
+// of 1024 SIMDs idle and the rest at the longest item.  Bound there by the
+// quarters' operand work (eight MFMAs a ray for one evaluation of its rows).
 template <int kPrec>
-__global__ __launch_bounds__(gemm_threads<kPrec>(), gemm_waves_per_simd<kPrec>()) void k_psf_gemm_batch(
+__global__ __launch_bounds__(64, 1) void k_psf_gemm_batch(
     const float* __restrict__ params, const float* __restrict__ rot,
-    const WorkItem* __restrict__ items,
-    const int* __restrict__ nitems_ptr, int tiles_i, int tiles, int nx, int ny, int nxp,
-    int nyp, float* __restrict__ partial)
+    const WorkItem* __restrict__ items, const int* __restrict__ nitems_ptr,
+    unsigned long long* __restrict__ queue, int tiles_i, int tiles, int nx, int ny, int nxp, int nyp,
+    int simds, float* __restrict__ partial)
 {
-    const int64_t nwork = (int64_t)(*nitems_ptr) * tiles;
-    for (int64_t wk = blockIdx.x; wk < nwork; wk += gridDim.x) {
-        const int item = (int)(wk / tiles);
-        const int tile = (int)(wk % tiles);
-        const WorkItem it = items[item];
-        psf_tile<kPrec>(params, rot, it.r0, it.r1, (tile % tiles_i) * kTile, (tile / tiles_i) * kTile,
-                        nx, ny, nyp, partial + (int64_t)item * nxp * nyp * 2);
+    constexpr int kHalves = gemm_cb<kPrec>() == 4 ? 2 : 4;       // units of a tile
+    const int nitems = *nitems_ptr;
+    const bool quarters = kPrec == BT_PSF_FP32 && (int64_t)nitems * tiles * kHalves < 2 * simds;
+    const int parts = quarters ? 2 * kHalves : kHalves;
+    const int64_t nwork = (int64_t)nitems * tiles * parts;
+    for (;;) {
+        unsigned long long next = 0;
+        if (threadIdx.x == 0) next = atomicAdd(queue, 1ull);
+        const int64_t u =
+            (int64_t)((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(next >> 32)) << 32 |
+                      (uint32_t)__builtin_amdgcn_readfirstlane((int)next));
+        if (u >= nwork) return;                  // every wave gets here
+        const int part = (int)(u % parts), tile = (int)(u / parts % tiles);
+        const WorkItem it = items[u / parts / tiles];
+        float* const out = partial + (int64_t)it.place * nxp * nyp * 2;
+        const int ti = (tile % tiles_i) * kTile, tj = (tile / tiles_i) * kTile;
+        if constexpr (kPrec == BT_PSF_FP32) {
+            if (quarters) {
+                if (part < kHalves)
+                    psf_tile<kPrec, 1>(params, rot, it.r0, it.r1, ti, tj, part, nx, ny, nyp, out);
+                else
+                    psf_tile<kPrec, 2>(params, rot, it.r0, it.r1, ti, tj, part - kHalves, nx, ny,
+                                       nyp, out);
+                continue;
+            }
+        }
+        psf_tile<kPrec, 0>(params, rot, it.r0, it.r1, ti, tj, part, nx, ny, nyp, out);
     }
 }
 
-// amp[s][j][i] = sum over the segment's items of partial[item][i][j], FP64,
-// in the fixed order of reduce_splits.
+// amp[s][j][i] = sum over the segment's items of partial[item][i][j], FP64.
+// One lane per pixel where segments and pixels fill the chip by themselves
+// (a segment's few items in item order, four reads in flight), else the
+// lanes of reduce_splits.
+template <int L>
 __global__ __launch_bounds__(kBlock) void k_psf_reduce_batch(
     const float* __restrict__ partial, const SegRange* __restrict__ ranges, int nseg, int nx,
     int ny, int nxp, int nyp, int cap, double* __restrict__ amp)
 {
+    constexpr int kPix = L == 1 ? kBlock : kRedPix;
     const int64_t npix = (int64_t)nx * ny;
-    const int64_t blocks_per_seg = (npix + kRedPix - 1) / kRedPix;
+    const int64_t blocks_per_seg = (npix + kPix - 1) / kPix;
     const int sg = (int)(blockIdx.x / blocks_per_seg);
-    const int64_t q = (int64_t)(blockIdx.x % blocks_per_seg) * kRedPix + threadIdx.x % kRedPix;
+    const int64_t q = (int64_t)(blockIdx.x % blocks_per_seg) * kPix + threadIdx.x % kPix;
     const bool live = q < npix;
     const int i = live ? (int)(q / ny) : 0, j = live ? (int)(q % ny) : 0;
     const SegRange r = ranges[sg];
     const int last = min(r.first + r.items, cap);
     const float2* p = reinterpret_cast<const float2*>(partial) + ((int64_t)i * nyp + j);
-    reduce_splits(p, (int64_t)nxp * nyp, r.first, last, live,
-                  amp + 2 * ((int64_t)sg * npix + (int64_t)j * nx + i));
+    double* const out = amp + 2 * ((int64_t)sg * npix + (int64_t)j * nx + i);
+    const int64_t stride = (int64_t)nxp * nyp;
+    if constexpr (L > 1) {
+        reduce_splits<L>(p, stride, r.first, last, live, out);
+    } else if (live) {
+        double re = 0.0, im = 0.0;
+#pragma unroll 4
+        for (int k = r.first; k < last; k++) {
+            const float2 v = p[k * stride];
+            re += (double)v.x;
+            im += (double)v.y;
+        }
+        out[0] = re;
+        out[1] = im;
+    }
 }
 
 struct GemmLayout {
@@ -983,12 +1074,22 @@ int bt::huygens_gemm_launch(bt_rays rays, const double* p0, const double* a1,
                            L.tiles_i, L.ksplit, L.nxp, L.nyp, partial);
     rc = check_launch("bt_huygens_gemm(mfma)");
     if (rc) return rc;
-    hipLaunchKernelGGL(k_psf_reduce, dim3((unsigned)(((int64_t)nx * ny + kRedPix - 1) / kRedPix)),
-                       dim3(kBlock), 0, s, partial, L.ksplit, nx, ny, L.nxp, L.nyp, amp_out);
+    // few pixels and many splits: more lanes per pixel (see reduce_splits)
+    const dim3 red((unsigned)(((int64_t)nx * ny + kRedPix - 1) / kRedPix));
+    if (L.ksplit >= 128 && red.x <= 1024)
+        hipLaunchKernelGGL(k_psf_reduce<32>, red, dim3(32 * kRedPix), 0, s, partial, L.ksplit, nx,
+                           ny, L.nxp, L.nyp, amp_out);
+    else
+        hipLaunchKernelGGL(k_psf_reduce<8>, red, dim3(8 * kRedPix), 0, s, partial, L.ksplit, nx,
+                           ny, L.nxp, L.nyp, amp_out);
     return check_launch("bt_huygens_gemm(reduce)");
 }
 
 namespace bt {
+
+// Workgroups of the GEMM kernels that run at a time: two on each CU (two waves
+// of one per SIMD).
+constexpr int kGemmSlots = 512;
 
 struct BatchLayout {
     int64_t nblocks, cap;
@@ -1002,9 +1103,9 @@ BatchLayout batch_layout(int64_t n, int nseg, int nx, int ny, int chunk)
     BatchLayout L;
     L.nblocks = (n + kBlock - 1) / kBlock;
     if (L.nblocks < 1) L.nblocks = 1;
-    L.cap = (n + chunk - 1) / chunk + nseg;
     L.tiles_i = (nx + kTile - 1) / kTile;
     L.tiles_j = (ny + kTile - 1) / kTile;
+    L.cap = (n + chunk - 1) / chunk + nseg;
     L.nxp = L.tiles_i * kTile;
     L.nyp = L.tiles_j * kTile;
     auto align = [](int64_t v) { return (v + 255) & ~(int64_t)255; };
@@ -1014,7 +1115,7 @@ BatchLayout batch_layout(int64_t n, int nseg, int nx, int ny, int chunk)
     L.off_offsets = off; off = align(off + (L.nblocks + 1) * (int64_t)sizeof(int));
     L.off_ranges = off;  off = align(off + nseg * (int64_t)sizeof(SegRange));
     L.off_items = off;   off = align(off + L.cap * (int64_t)sizeof(WorkItem));
-    L.off_nitems = off;  off = align(off + (int64_t)sizeof(int));
+    L.off_nitems = off;  off = align(off + 2 * (int64_t)sizeof(int64_t));   // and the queue
     L.off_params = off;
     off = align(off + (n + kRayGroup) * (kRayStride + kRotStride) * (int64_t)sizeof(float));
     L.off_partial = off; off = align(off + L.cap * L.nxp * L.nyp * 2 * (int64_t)sizeof(float));
@@ -1061,6 +1162,7 @@ extern "C" int bt_huygens_batch(bt_rays rays, const bt_psf_segment* segments, in
     SegRange* ranges = reinterpret_cast<SegRange*>(ws + L.off_ranges);
     WorkItem* items = reinterpret_cast<WorkItem*>(ws + L.off_items);
     int* nitems = reinterpret_cast<int*>(ws + L.off_nitems);
+    auto* queue = reinterpret_cast<unsigned long long*>(ws + L.off_nitems + sizeof(int64_t));
     float* params = reinterpret_cast<float*>(ws + L.off_params);
     float* rot = params + (rays.n + kRayGroup) * kRayStride;
     float* partial = reinterpret_cast<float*>(ws + L.off_partial);
@@ -1091,28 +1193,37 @@ extern "C" int bt_huygens_batch(bt_rays rays, const bt_psf_segment* segments, in
         rc = check_launch("bt_huygens_batch(prep)");
         if (rc) return rc;
     }
-    hipLaunchKernelGGL(k_psf_seg_ranges, dim3((nseg + kBlock - 1) / kBlock), dim3(kBlock), 0, s,
-                       rays, segments, nseg, ignore_vignetted, offsets, chunk, ranges);
+    hipLaunchKernelGGL(k_psf_seg_ranges, dim3((nseg + kBlock / 64 - 1) / (kBlock / 64)),
+                       dim3(kBlock), 0, s, rays, segments, nseg, ignore_vignetted, offsets, chunk,
+                       ranges);
     rc = check_launch("bt_huygens_batch(ranges)");
     if (rc) return rc;
     hipLaunchKernelGGL(k_psf_items, dim3(1), dim3(kScanThreads), 0, s, ranges, nseg, chunk,
-                       (int)L.cap, items, nitems);
+                       (int)L.cap, items, nitems, queue);
     rc = check_launch("bt_huygens_batch(items)");
     if (rc) return rc;
-    const int grid = nwg > 0 ? nwg : 512;
+    // nwg counts workgroups of two waves
+    const int grid = 2 * (nwg > 0 ? nwg : kGemmSlots);
+    const int simds = 2 * kGemmSlots;
     const int tiles = L.tiles_i * L.tiles_j;
     if (precision == BT_PSF_FP32)
-        hipLaunchKernelGGL(k_psf_gemm_batch<BT_PSF_FP32>, dim3(grid),
-                           dim3(gemm_threads<BT_PSF_FP32>()), 0, s, params,
-                           rot, items, nitems, L.tiles_i, tiles, nx, ny, L.nxp, L.nyp, partial);
+        hipLaunchKernelGGL(k_psf_gemm_batch<BT_PSF_FP32>, dim3(grid), dim3(64), 0, s, params, rot,
+                           items, nitems, queue, L.tiles_i, tiles, nx, ny, L.nxp, L.nyp,
+                           simds, partial);
     else
-        hipLaunchKernelGGL(k_psf_gemm_batch<BT_PSF_BF16X3>, dim3(grid),
-                           dim3(gemm_threads<BT_PSF_BF16X3>()), 0, s, params,
-                           rot, items, nitems, L.tiles_i, tiles, nx, ny, L.nxp, L.nyp, partial);
+        hipLaunchKernelGGL(k_psf_gemm_batch<BT_PSF_BF16X3>, dim3(grid), dim3(64), 0, s, params,
+                           rot, items, nitems, queue, L.tiles_i, tiles, nx, ny, L.nxp, L.nyp,
+                           simds, partial);
     rc = check_launch("bt_huygens_batch(mfma)");
     if (rc) return rc;
-    const int64_t red_blocks = (((int64_t)nx * ny + kRedPix - 1) / kRedPix) * nseg;
-    hipLaunchKernelGGL(k_psf_reduce_batch, dim3((unsigned)red_blocks), dim3(kBlock), 0, s, partial,
-                       ranges, nseg, nx, ny, L.nxp, L.nyp, (int)L.cap, amp_out);
+    const int64_t npix = (int64_t)nx * ny;
+    if (npix * nseg >= ((int64_t)1 << 18))          // 4096 waves, four per SIMD
+        hipLaunchKernelGGL(k_psf_reduce_batch<1>,
+                           dim3((unsigned)((npix + kBlock - 1) / kBlock * nseg)), dim3(kBlock), 0,
+                           s, partial, ranges, nseg, nx, ny, L.nxp, L.nyp, (int)L.cap, amp_out);
+    else
+        hipLaunchKernelGGL(k_psf_reduce_batch<8>,
+                           dim3((unsigned)((npix + kRedPix - 1) / kRedPix * nseg)), dim3(kBlock),
+                           0, s, partial, ranges, nseg, nx, ny, L.nxp, L.nyp, (int)L.cap, amp_out);
     return check_launch("bt_huygens_batch(reduce)");
 }

@@ -632,8 +632,9 @@ int bt_huygens_gemm_noalloc(bt_rays rays, const double* p0, const double* a1,
  * The segment table lives in device memory, so one call can be captured in a
  * HIP graph and replayed on new ray data: no host synchronisation, no
  * allocation, no memset.  Rays are summed in work items of `chunk` rays (a
- * multiple of 8) by `nwg` persistent workgroups (0: 512) in a fixed
- * assignment; items of one segment are added in FP64 in item order.
+ * multiple of 8) that two waves for each of `nwg` (0: 512) take from a queue;
+ * a result does not depend on who takes an item, and the items of one segment
+ * are added in FP64 in a fixed order.
  * `amp_out` receives [nseg][ny][nx][2] complex128.                         */
 typedef struct bt_psf_segment {
     int64_t begin, end;
