@@ -113,8 +113,13 @@ def huygensPSF(optic, theta_x, theta_y, wavelength, projection='postel', nx=None
     dirCos = fieldToDirCos(theta_x, theta_y, projection=projection)
     rays = RayVector.asGrid(optic=optic, wavelength=wavelength, dirCos=dirCos, nx=nx)
     optic.trace(rays)
-    point = _reference_point(rays, nx, reference)
-    time = float(rays.torch("t")[0].item())
+    if reference == 'chief':             # the point and the first ray's time in one read-back
+        k = _chief_index(nx)
+        *point, time = torch.stack([rays.torch(c)[i] for c, i in (
+            ("x", k), ("y", k), ("z", k), ("t", 0))]).tolist()
+    else:
+        point = _reference_point(rays, nx, reference)
+        time = float(rays.torch("t")[0].item())
     n = nxOut * pad_factor
     amp = huygens_amplitudes(rays, point, primitiveX, n, n, time, True, method, precision)
     return Lattice(np.abs(amp) ** 2, primitiveX)

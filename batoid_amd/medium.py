@@ -45,6 +45,14 @@ class ConstMedium(Medium):
     def __init__(self, n):
         self.n = n
 
+    def getN(self, wavelength):
+        """``n``; for a plain number without asking the GPU, whose answer is
+        the record's ``n`` itself (an upload, a launch and a read-back less in
+        every ray generation)."""
+        if isinstance(wavelength, (int, float)):
+            return float(self.n)
+        return Medium.getN(self, wavelength)
+
     def _record(self):
         return _rec(_lib.MED_CONST, [self.n]), (None, None)
 

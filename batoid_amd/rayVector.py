@@ -385,7 +385,6 @@ class RayVector:
         gen.rot[:] = [float(v) for v in rot.ravel()]
         gen.vv[:] = [float(v) for v in vv]
         gen.wavelength = float(wavelength)
-        dev = _device.device()
         fluxd = None
         if isinstance(flux, Real):
             gen.flux0 = float(flux)
@@ -398,10 +397,9 @@ class RayVector:
             rv = out
             rv.coordSys = coordSys
         else:
-            cols = {k: torch.empty(npts, dtype=torch.float64, device=dev) for k in _FCOLS}
-            for k in _BCOLS:
-                cols[k] = torch.empty(npts, dtype=torch.uint8, device=dev)
-            rv = cls._directInit(cols, coordSys)
+            # one allocation: copy() of the rays is then one device copy (5 us
+            # of host time for each of eleven columns before)
+            rv = cls._empty(npts, coordSys)
         # inputs (tables, points, fluxes) are torch tensors on the current
         # stream: their memory is not reused before this launch has read it
         _lib.call("bt_generate_rays", ctypes.byref(gen), rv._rays, _device.stream())
@@ -518,7 +516,7 @@ class RayVector:
         args = (stopSurface, coordSys, wavelength, medium, backDist, source, dirCos, flux)
         gen = _lib.BtRaygen()
         if nrandom is None:
-            npts, _tables = cls._polar_tables(gen, outer, inner, nrad, naz, kfold)
+            npts, _table = cls._polar_tables(gen, outer, inner, nrad, naz, kfold)
             return cls._generate(gen, npts, *args)
         if rng is None:
             rng = np.random.default_rng()
@@ -538,17 +536,19 @@ class RayVector:
         """Hexapolar rings (utils.py:512-531) as the device ring table of a
         POLAR generator: ray j of ring k sits at th = j * (2 pi / nphi_k),
         numpy's linspace(0, 2 pi, nphi_k, endpoint=False).  Returns the ray
-        count and the device tables (keep them alive until the launch)."""
+        count and the device table (keep it alive until the launch)."""
         rhos, nphis, dth = _hexapolar_rings(outer, inner, nrad, naz, kfold)
         off = np.zeros(len(nphis) + 1, dtype=np.int64)
         off[1:] = np.cumsum(nphis)
-        off_d = torch.from_numpy(off).to(_device.device())
-        rho_d, dth_d = _device.f64(rhos), _device.f64(dth)
+        # the three tables in one upload (each waits for the stream)
+        nring = len(nphis)
+        table = _device.f64(np.concatenate([off.view(np.float64), rhos, dth]))
         gen.pattern = _lib.GEN_POLAR
-        gen.nring = len(nphis)
-        gen.ring_off, gen.ring_rho, gen.ring_dth = (
-            off_d.data_ptr(), rho_d.data_ptr(), dth_d.data_ptr())
-        return int(off[-1]), (off_d, rho_d, dth_d)
+        gen.nring = nring
+        gen.ring_off = table.data_ptr()
+        gen.ring_rho = gen.ring_off + 8 * (nring + 1)
+        gen.ring_dth = gen.ring_rho + 8 * nring
+        return int(off[-1]), table
 
     @classmethod
     def asSpokes(cls, optic=None, backDist=None, medium=None, stopSurface=None,

@@ -378,3 +378,10 @@ def test_horner_trim_layout():
     one = _horner_trim([(np.array([[3.0]]), 1, 1), (np.zeros((1, 1)), 0, 0),
                         (np.zeros((1, 1)), 0, 0)])
     assert list(one) == [0, 1, -1, -1]
+
+
+@pytest.mark.parametrize("wavelength", [0, 5e-7, np.float64(5e-7), float("nan")])
+def test_constant_index_on_the_host(wavelength):
+    """A constant medium's index at one plain number is its own, exactly."""
+    n = bt.ConstMedium(np.nextafter(1.1, 2)).getN(wavelength)
+    assert type(n) is float and n == np.nextafter(1.1, 2)
