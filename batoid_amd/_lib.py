@@ -13,6 +13,8 @@ import numpy as np
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libbatoid_amd.so")
 
+POLY_STREAMS = 1             # BtSurface.flags of a POLYNOMIAL: a3 holds streams
+
 c_double_p = ctypes.POINTER(ctypes.c_double)
 c_u8_p = ctypes.POINTER(ctypes.c_uint8)
 

@@ -277,6 +277,32 @@ def _horner_trim(tables):
     return np.array(out, dtype=np.int32)
 
 
+def _horner_streams(tables, trim):
+    """The device's streams of 2-D Horner tables trimmed to ``trim``
+    (include/batoid_amd.h, POLYNOMIAL): ``trim`` itself and what follows it in
+    a3, as one int32 array.  A table of no coefficients or of more than 64
+    quads (a full 16 x 16 table) has no stream."""
+    heads = np.zeros(3, dtype=[("nquad", "<i4"), ("first", "<i4"), ("row_ends", "<u8")])
+    data, k = [], 0
+    for head, (flat, nx, ny) in zip(heads, tables):
+        last, lens = int(trim[k]), trim[k + 1:k + 1 + ny]
+        k += 1 + ny
+        flat = np.ascontiguousarray(flat, dtype=np.float64).ravel()
+        quads = [max(-(-int(lens[i]) // 4), 1) for i in range(last, -1, -1)]
+        if not 0 < sum(quads) <= 64:
+            continue
+        head["nquad"] = sum(quads)
+        head["first"] = len(data)
+        head["row_ends"] = sum(1 << int(q - 1) for q in np.cumsum(quads))
+        for i, q in zip(range(last, -1, -1), quads):
+            row = flat[i * nx:i * nx + int(lens[i])][::-1]
+            data += [0.0] * (4 * q - len(row)) + row.tolist()
+    data += [0.0] * 4
+    pad = np.zeros(-len(trim) % 16, dtype=np.int32)
+    return np.concatenate([trim, pad, heads.view(np.int32), np.zeros(4, dtype=np.int32),
+                           np.array(data, dtype=np.float64).view(np.int32)])
+
+
 class Zernike(Surface):
     """Annular Zernike series sum_j coef[j] Z_j(x/R_outer, y/R_outer) in
     Noll order (surface.py:433-518), evaluated as a 2-D polynomial
@@ -296,10 +322,12 @@ class Zernike(Surface):
     def _leaf_record(self):
         c = self._xycoef
         n1, n2 = c.shape
-        trim = _horner_trim([(c, n1, n2), (self._xycoef_gradx, n1 - 1, n2 - 1),
-                             (self._xycoef_grady, n1 - 1, n2 - 1)])
-        return (_rec(_lib.POLYNOMIAL, [self.x_origin, self.y_origin], n1=n1, n2=n2),
-                (c, self._xycoef_gradx, self._xycoef_grady, trim))
+        tables = [(c, n1, n2), (self._xycoef_gradx, n1 - 1, n2 - 1),
+                  (self._xycoef_grady, n1 - 1, n2 - 1)]
+        return (_rec(_lib.POLYNOMIAL, [self.x_origin, self.y_origin], n1=n1, n2=n2,
+                     flags=_lib.POLY_STREAMS),
+                (c, self._xycoef_gradx, self._xycoef_grady,
+                 _horner_streams(tables, _horner_trim(tables))))
 
     def __hash__(self):
         return hash(("batoid.Zernike", tuple(self.coef), self.R_outer, self.R_inner,

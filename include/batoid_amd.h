@@ -83,6 +83,14 @@ typedef struct bt_rays {
  *                +0.0 (-1 if none), then each row's length up to its last
  *                such coefficient (1 + n2, n2, n2 entries).  Evaluation
  *                skips the +0.0 runs it marks, with bit-identical results.
+ *                flags & BT_POLY_STREAMS: a3 goes on, at the next multiple
+ *                of 64 bytes, with three bt_poly_stream (one per table) in
+ *                64 bytes, then with the streams they point into: each
+ *                table's coefficients in the order of evaluation, rows from
+ *                the trim table's last down, in a row from its last down,
+ *                +0.0 in front to a multiple of four (a row of only +0.0 is
+ *                one quad of them); one quad more follows the last stream.
+ *                Results are again bit-identical.
  *   SUM          nchild children follow; n1 = records below   sum.cpp:23-56
  */
 enum bt_surface_kind {
@@ -90,6 +98,14 @@ enum bt_surface_kind {
     BT_ASPHERE = 4, BT_TILTED = 5, BT_BICUBIC = 6, BT_POLYNOMIAL = 7,
     BT_SUM = 8
 };
+
+#define BT_POLY_STREAMS 1
+
+typedef struct bt_poly_stream {
+    int32_t nquad;            /* quads of coefficients; 0: table without stream */
+    int32_t first;            /* its first coefficient's index in the streams */
+    uint64_t row_ends;        /* bit k: quad k ends a row (nquad <= 64) */
+} bt_poly_stream;
 
 typedef struct bt_surface {
     int32_t kind;
