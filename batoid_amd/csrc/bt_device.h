@@ -320,38 +320,47 @@ BT_DEV void table_grad(SurfPtr s, double x, double y,
 // ---------------------------------------------------------------------------
 // A table's steps as one stream of quads (bt_poly_stream): rows from the last
 // down, each row's coefficients from its last down, with +0.0 in front to a
-// multiple of four; bit k of `row_ends` says that a row ends with quad k.  The
-// argument below makes the steps over the +0.0 in front exact.  A quad is one
-// 32-byte scalar load, issued while the quad before it is used (the stream
-// has one quad more than its steps): the loop over single coefficients waits
-// for a load and runs eight scalar instructions for its two of FP64, which
-// left the Sum kernels' SIMDs idle a third to two thirds of the time.  Plan
-// kernels before and after, one card, same clocks: 704 -> 587 us (1e6 rays,
-// three perturbed mirrors), 1071 -> 934 (3e6, conic start), 461 -> 311 (3e5,
-// freeform), 764 -> 635 (the batched trace of 1.1e6).  The two gradients'
-// streams in one loop: no faster on the first, 9 % slower on the freeform
-// (scalar registers spill).
-BT_DEV double horner2d_stream(double x, double y, CoefPtr c, int nquad, uint64_t row_ends)
+// multiple of four; bit k of `row_ends` says that a row ends with quad k, and
+// its highest bit is the last quad's.  The argument below makes the steps over
+// the +0.0 in front exact.  A quad is one 32-byte scalar load, issued while the
+// quad before it is used (the stream has one quad more than its steps); two
+// quads per pass, so that no register is copied.  The loop over single
+// coefficients waits for a load and runs eight scalar instructions for its two
+// of FP64, which left the Sum kernels' SIMDs idle a third to two thirds of the
+// time.  Plan kernels with it, with one quad per pass and with two, same card
+// and clocks: 704, 587, 573 us (1e6 rays, three perturbed mirrors), 1071, 934,
+// 916 (3e6, conic start), 461, 311, 303 (3e5, freeform), 764, 635, 623 (the
+// batched trace of 1.1e6).  The two gradients' streams side by side in one loop,
+// or all three tables' as one stream, were 3 to 9 % slower on the freeform
+// (scalar registers spill; more scalar work per quad).
+BT_DEV double horner2d_stream(double x, double y, CoefPtr c, uint64_t row_ends)
 {
     double r = 0.0, h = 0.0;
-    double c0 = c[0], c1 = c[1], c2 = c[2], c3 = c[3];
-    __builtin_amdgcn_s_waitcnt(0xc07f);          // lgkmcnt(0): else each pass waits up front
-    for (int k = 0; k < nquad; k++) {
-        c += 4;
-        const double d0 = c[0], d1 = c[1], d2 = c[2], d3 = c[3];
-        __builtin_amdgcn_sched_barrier(0);
-        h *= y; h += c0;
-        h *= y; h += c1;
-        h *= y; h += c2;
-        h *= y; h += c3;
+    auto quad = [&](double k0, double k1, double k2, double k3) {
+        h *= y; h += k0;
+        h *= y; h += k1;
+        h *= y; h += k2;
+        h *= y; h += k3;
         if (row_ends & 1) {
-            asm volatile("");                        // a branch, not six selects
+            asm volatile("");                    // a branch, not six selects
             r *= x;
             r += h;
             h = 0.0;
         }
         row_ends >>= 1;
-        c0 = d0; c1 = d1; c2 = d2; c3 = d3;
+    };
+    double c0 = c[0], c1 = c[1], c2 = c[2], c3 = c[3];
+    __builtin_amdgcn_s_waitcnt(0xc07f);          // lgkmcnt(0): else each pass waits up front
+    for (;;) {
+        const double d0 = c[4], d1 = c[5], d2 = c[6], d3 = c[7];
+        __builtin_amdgcn_sched_barrier(0);
+        quad(c0, c1, c2, c3);
+        if (!row_ends) break;
+        c0 = c[8]; c1 = c[9]; c2 = c[10]; c3 = c[11];
+        c += 8;
+        __builtin_amdgcn_sched_barrier(0);
+        quad(d0, d1, d2, d3);
+        if (!row_ends) break;
     }
     return r;
 }
@@ -391,10 +400,9 @@ BT_DEV double poly_table(SurfPtr s, int which, double u, double v, bool finite)
         if (s->flags & BT_POLY_STREAMS) {
             const TrimPtr head = trim + ((1 + 3*n2 + 15) & ~15);
             const StreamPtr st = (StreamPtr)head + which;
-            const int nquad = st->nquad;
-            if (nquad > 0)
-                return horner2d_stream(u, v, (CoefPtr)(head + 16) + st->first, nquad,
-                                       st->row_ends);
+            const uint64_t row_ends = st->row_ends;
+            if (row_ends)
+                return horner2d_stream(u, v, (CoefPtr)(head + 16) + st->first, row_ends);
         }
         if (which > 0) trim += 1 + n2 + (which - 1)*n2;
     }

@@ -104,7 +104,8 @@ enum bt_surface_kind {
 typedef struct bt_poly_stream {
     int32_t nquad;            /* quads of coefficients; 0: table without stream */
     int32_t first;            /* its first coefficient's index in the streams */
-    uint64_t row_ends;        /* bit k: quad k ends a row (nquad <= 64) */
+    uint64_t row_ends;        /* bit k: quad k ends a row, the last too
+                                 (nquad <= 64); 0: table without stream */
 } bt_poly_stream;
 
 typedef struct bt_surface {
