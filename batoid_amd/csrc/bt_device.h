@@ -1685,6 +1685,20 @@ struct Arrival {
     NormalMemo memo;
 };
 
+// A rotation by nothing: the unit matrix, zeros of either sign (tested on the
+// scalar unit).  Its products are exact, so 12 FMAs give the bits of the 18
+// products and 12 sums, signed zeros and NaNs included.  Only in the kernels
+// of analytic surfaces, which issue bounds: 1786 -> 1753 us for 1e7 rays
+// through twelve Interfaces; the freeform kernel was 2 % slower with it.
+template <class Frame>
+BT_DEV bool unrotated(Frame m)
+{
+    auto bits = [](double v) { return __builtin_bit_cast(uint64_t, v); };
+    const uint64_t off = bits(m[1]) | bits(m[2]) | bits(m[3]) | bits(m[5]) | bits(m[6]) | bits(m[7]);
+    const uint64_t dia = (bits(m[0]) ^ bits(1.0)) | (bits(m[4]) ^ bits(1.0)) | (bits(m[8]) ^ bits(1.0));
+    return ((off << 1) | dia) == 0;
+}
+
 // Frame change and intersection; false where the ray misses the surface.
 template <int K, bool kPlain, class Frame>
 BT_DEV bool arrive(Frame dr, Frame drot,
@@ -1694,12 +1708,21 @@ BT_DEV bool arrive(Frame dr, Frame drot,
     double dx = r.x-dr[0];
     double dy = r.y-dr[1];
     double dz = r.z-dr[2];
-    a.x = dx*drot[0] + dy*drot[3] + dz*drot[6];
-    a.y = dx*drot[1] + dy*drot[4] + dz*drot[7];
-    a.z = dx*drot[2] + dy*drot[5] + dz*drot[8];
-    a.vx = r.vx*drot[0] + r.vy*drot[3] + r.vz*drot[6];
-    a.vy = r.vx*drot[1] + r.vy*drot[4] + r.vz*drot[7];
-    a.vz = r.vx*drot[2] + r.vy*drot[5] + r.vz*drot[8];
+    if (K == kKindsAnalytic && unrotated(drot)) {
+        a.x = __builtin_fma(dz, drot[6], __builtin_fma(dy, drot[3], dx));
+        a.y = __builtin_fma(dz, drot[7], __builtin_fma(dx, drot[1], dy));
+        a.z = __builtin_fma(dy, drot[5], __builtin_fma(dx, drot[2], dz));
+        a.vx = __builtin_fma(r.vz, drot[6], __builtin_fma(r.vy, drot[3], r.vx));
+        a.vy = __builtin_fma(r.vz, drot[7], __builtin_fma(r.vx, drot[1], r.vy));
+        a.vz = __builtin_fma(r.vy, drot[5], __builtin_fma(r.vx, drot[2], r.vz));
+    } else {
+        a.x = dx*drot[0] + dy*drot[3] + dz*drot[6];
+        a.y = dx*drot[1] + dy*drot[4] + dz*drot[7];
+        a.z = dx*drot[2] + dy*drot[5] + dz*drot[8];
+        a.vx = r.vx*drot[0] + r.vy*drot[3] + r.vz*drot[6];
+        a.vy = r.vx*drot[1] + r.vy*drot[4] + r.vz*drot[7];
+        a.vz = r.vx*drot[2] + r.vy*drot[5] + r.vz*drot[8];
+    }
     a.t = r.t;
     a.dt = 0.0;
     a.memo.ok = false;
