@@ -50,9 +50,11 @@ __device__ __forceinline__ void mlp_features(StepPtr st, SurfPtr surf, const Ray
 
 // Waves per SIMD: the analytic-kinds kernels of modes 0 and 1 are held to
 // six (79 and 80 VGPRs), the Sum(Asphere, Polynomial, Bicubic) kernels to
-// four (128 VGPRs; mode 0 spills 20 words outside its Newton loops), the
+// four (128 VGPRs; mode 0 spills 18 words outside its Newton loops), the
 // others of mode 0 to four and of modes 1 and 2 to three (left alone the
-// compiler would settle for two).
+// compiler would settle for two).  Mode 0 at three, four and five waves: 621,
+// 573, 655 us (1e6 rays, three perturbed mirrors), 320, 304, 372 (3e5,
+// freeform); the conic start on the first, 3e6 rays: 1002, 918, 1305.
 // Networks a plan kernel keeps in LDS (45 KB per workgroup).
 constexpr int kMlpLds = 4;
 
