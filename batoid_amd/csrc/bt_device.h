@@ -515,6 +515,10 @@ BT_DEV void table_point(SurfPtr s, double x, double y, double& sag, double& nx,
 // on the Sum kernels, whose scalar registers are short.)
 BT_DEV double even_terms(CoefPtr c, int n, double result, double term, double r2)
 {
+    // n anew for each evaluation: a test of it shared by two Newton loops is
+    // kept as a mask of the lanes active in the first, which may have none in
+    // common with those of the second, and then no terms reads as some
+    asm volatile("" : "+s"(n));
     for (int i = 0; i < n; i++) {
         result += c[i]*term;
         term *= r2;

@@ -158,21 +158,18 @@ def trace_split(optic, rv, reverse, minFlux, bound):
         if not s.leaves:                 # a chain that ends unseen: up to its last split
             while s.steps and s.steps[-1][2] is None:
                 s.steps.pop()
-    # a set that nothing comes of is not written
+    # a set that nothing comes of is not written (a set's reflected parts stand
+    # behind it in the list)
     live = set()
-
-    def needed(s):
+    for s in reversed(sets):
         ok = s.leaves
         for k, (item, rev, split) in enumerate(s.steps):
-            if split is not None:
-                if needed(split):
-                    ok = True
-                else:
-                    s.steps[k] = (item, rev, None)
+            if split in live:
+                ok = True
+            else:
+                s.steps[k] = (item, rev, None)
         if ok:
             live.add(s)
-        return ok
-    needed(root)
     rv.path = path + [item.name for item, _, _ in root.steps]
     frames, records, kinds = {}, {}, {}
     n = len(rv)

@@ -69,3 +69,25 @@ def test_chains_equal_counted_rounds(monkeypatch, name, n, minFlux):
             assert len(a) == len(b) and a.coordSys == b.coordSys
             assert_cols_identical(host(a), host(b), what=f"{name} {'/'.join(a.path)}")
     assert n < 200 or sum(map(len, got)) > 3
+
+
+def test_many_turns_back(monkeypatch):
+    """A thousand reflections between two windows: as many sets, one after the
+    other, and no recursion."""
+    glass = [bt.RefractiveInterface(
+        bt.Plane(), name=name, inMedium=bt.ConstMedium(1.0), outMedium=bt.ConstMedium(1.0),
+        coordSys=bt.CoordSys(origin=[0, 0, z])) for name, z in (("A", 0.0), ("B", 0.1))]
+    optic = coated(bt.CompoundOptic(glass, name="o", inMedium=bt.ConstMedium(1.0),
+                                    outMedium=bt.ConstMedium(1.0)), r=0.98)
+    rays = bt.RayVector(x=[0.0, 0.01], y=[0.0, 0.02], z=[-1.0, -1.0], vx=[0.0, 1e-5],
+                        vy=[0.0, 0.0], vz=[1.0, 1.0])
+    minFlux = 0.02 * 0.02 * 0.98**1200
+    got = optic.traceSplit(rays.copy(), minFlux=minFlux)
+    assert max(len(r.path) for r in got[0] + got[1]) > 1100
+    with monkeypatch.context() as mp:
+        mp.setattr(bt.CompoundOptic, "_flux_bound", lambda self, rv, m: None)
+        want = optic.traceSplit(rays.copy(), minFlux=minFlux)
+    for g, w in zip(got, want):
+        assert [r.path for r in g] == [r.path for r in w]
+        for a, b in zip(g, w):
+            assert_cols_identical(host(a), host(b))
