@@ -70,11 +70,15 @@ using TablePtr = const BT_GLOBAL double*;
 // per value noted: the compares and scalar masks of a test at each root cost
 // the plan kernel of the analytic surfaces 11 % (1.93 against 1.73 ms for
 // 1e7 rays through twelve interfaces).  What is noted:
-//  * every argument of a root (a zero, a negative one, an overflow, a NaN);
+//  * arguments of roots (a zero, a negative one, one below 2^-767, an
+//    overflow, a NaN) and denominators;
 //  * the exponents of a ray's x and y at each surface and of its final
-//    velocity: nothing nonzero below 2^-601, so that no remainder n - d q of a
-//    quotient underflows.  (A difference of two doubles is 0 or at least an
-//    ulp of theirs, so tiny values come only from tiny values.)
+//    velocity: nothing nonzero below 2^-383.  So x*x + y*y, whose root is
+//    taken without a note of its own, is 0 (a NaN slope follows, which is
+//    noted) or at least 2^-766, and no remainder n - d q of a quotient
+//    underflows.  (A difference of two doubles is 0 or at least an ulp of
+//    theirs, so tiny values come only from tiny values; where a Newton
+//    iterate alone is tiny, its slopes are lost beside the other terms.)
 // One pair of operands is given up: n a power of two over a d whose
 // significand is all ones, where a reciprocal refined from a root's h rounds
 // the quotient down an ulp.
@@ -83,31 +87,26 @@ struct Range {
     uint32_t high = 0;           // largest high word noted
     int32_t low = 0;             // smallest exponent noted
 
-    // w > 0 expected: an overflow, a NaN or a negative w is out of range
+    // w >= 1 expected: an overflow, a NaN or a negative w is out of range
     __device__ __forceinline__ void above(double w)
     {
         high = max(high, (uint32_t)__double2hiint(w));
     }
-    // as above, and zero too (the high word of a positive double below
-    // 2^-1022 is 0 only if it is below 2^-1042)
+    // as above, and what is below 2^-767 too: its high word wraps round
     __device__ __forceinline__ void positive(double w)
     {
-        high = max(high, (uint32_t)__double2hiint(w) - 1u);
-    }
-    __device__ __forceinline__ void positive(double w, double v)
-    {
-        high = max(max(high, (uint32_t)__double2hiint(w) - 1u),
-                   (uint32_t)__double2hiint(v) - 1u);
+        high = max(high, (uint32_t)__double2hiint(w) - ((1023u - 767u) << 20));
     }
     __device__ __forceinline__ void not_tiny(double a, double b)
     {
         low = min(min(low, __builtin_amdgcn_frexp_exp(a)), __builtin_amdgcn_frexp_exp(b));
     }
     __device__ __forceinline__ void leave() { high = ~0u; }
-    // below 2^601, and nothing nonzero below 2^-601
+    // roots' arguments from 2^-767 to 2^857, slopes' below 2^601, and nothing
+    // nonzero below 2^-383
     __device__ __forceinline__ bool plain() const
     {
-        return (high < ((1023u + 601u) << 20)) & (low >= -600);
+        return (high < ((1023u + 601u) << 20)) & (low >= -382);
     }
 };
 
