@@ -56,9 +56,15 @@ using TablePtr = const BT_GLOBAL double*;
 //    of v_rcp_f64 and 4), and quotients by one denominator (x/r and y/r, the
 //    velocity by an index) share one reciprocal: a quotient is then 3
 //    instructions instead of 11 (v_rcp_f64 alone takes four issue slots);
-//  * a reciprocal y that is within an ulp of 1/d makes q = n y,
-//    q + (n - d q) y the correctly rounded quotient, which is the division's
-//    own last step, so the bits are the division's.
+//  * from a reciprocal y of d in [1, 2) to 1/2 + e ulp, q = n y and then
+//    q + (n - d q) y is n/d correctly rounded (the division's own last step)
+//    for every n if d^2 (1 + 2 e) < 4: a quotient in [1, 2) is no closer than
+//    2^-105 / d to the midpoint of two doubles, and the error of y moves the
+//    sum by 2^-107 d (1 + 2 e) at most (in [1/2, 1) both are half as large).
+//    A Newton step from 2^-47 has e < 2^-41, which leaves the d within 2^11
+//    ulps below 2.  There every second 1/d lies a hair above a midpoint, and
+//    the step, whose error is to the lower side, may round it down:
+//    recip_root and recip_nearest see to these.
 // Every function of the trace exists in two forms.  The plain form (kPlain
 // true) runs these alone and notes in a Range what could have left their
 // range; a wave votes once on its lanes' Ranges, and only if one left it is
@@ -79,9 +85,6 @@ using TablePtr = const BT_GLOBAL double*;
 //    underflows.  (A difference of two doubles is 0 or at least an ulp of
 //    theirs, so tiny values come only from tiny values; where a Newton
 //    iterate alone is tiny, its slopes are lost beside the other terms.)
-// One pair of operands is given up: n a power of two over a d whose
-// significand is all ones, where a reciprocal refined from a root's h rounds
-// the quotient down an ulp.
 // ---------------------------------------------------------------------------
 struct Range {
     uint32_t high = 0;           // largest high word noted
@@ -137,8 +140,25 @@ BT_DEV double recip_refine(double d, double y0)
     return __builtin_fma(y0, __builtin_fma(-d, y0, 1.0), y0);
 }
 
-// 1/g to within an ulp for g = sqrt_plain(x, h).
-BT_DEV double recip_root(double g, double h) { return recip_refine(g, h + h); }
+// y with its last bit set.
+BT_DEV double odd(double y)
+{
+    return __longlong_as_double(__double_as_longlong(y) | 1);
+}
+
+// 1/g for quotients by g = sqrt_plain(x, h).  Next below a power of two h is
+// right to 2^-53, and g of all ones is the one whose reciprocal the step from
+// an even 2h rounds down (from 2h = 1/g rounded down it stays there).
+BT_DEV double recip_root(double g, double h) { return recip_refine(g, odd(h + h)); }
+
+// 1/d for quotients by any d, from y0 = 1/d to ~2^-46: a second step, whose
+// multiplier's last bit carries the one case (d of all ones) that it leaves on
+// a midpoint over it.
+BT_DEV double recip_nearest(double d, double y0)
+{
+    const double y = recip_refine(d, y0);
+    return __builtin_fma(__builtin_fma(-d, y, 1.0), odd(y), y);
+}
 
 // 1/d to within an ulp.
 BT_DEV double recip_plain(double d)
@@ -527,8 +547,8 @@ BT_DEV double even_terms(CoefPtr c, int n, double result, double term, double r2
 
 // Sag and / or normal of a Quadric (kAsphere false) or an Asphere (true) at
 // one point: quadric.cpp:18-39, asphere.cpp:37-62.  `inv`: 1/nz to an ulp,
-// or 0.  Bound by FP64 issue: the normal's three divisions and the reciprocal
-// of its third root come from the roots' own h here.
+// or 0.  Bound by FP64 issue: the normal's three divisions start from the
+// roots' own h here (the reciprocal of its third root does not: rsqrt_plain).
 template <bool kPlain, bool kAsphere, bool kSag, bool kNormal>
 BT_DEV void conic_point(SurfPtr s, double x, double y, double& sag, double& nx,
                         double& ny, double& nz, double& inv, Range& rg)
@@ -551,7 +571,7 @@ BT_DEV void conic_point(SurfPtr s, double x, double y, double& sag, double& nx,
             const double u = 1-r*r*cp1R2;
             const double d = R*sqrt_plain(u, hu);
             const double y0 = (hu + hu) * (R*s->p[3]);   // 1/sqrt(u) * (R * 1/R/R)
-            double dzdr = div_plain(r, d, recip_refine(d, y0));
+            double dzdr = div_plain(r, d, recip_nearest(d, y0));
             if constexpr (kAsphere) dzdr = even_terms((CoefPtr)s->a1, s->n1, dzdr, r, r*r);
             const double w = 1+dzdr*dzdr;
             rg.above(w);                                 // a NaN for r2 = 0 or u = 0
@@ -809,7 +829,9 @@ BT_DEV void leaf_point(SurfPtr s, double x, double y, double& sag,
     if constexpr (kNormal) leaf_normal<K, kPlain>(s, x, y, nx, ny, nz, inv, rg);
 }
 
-// sx += nx/nz, sy += ny/nz; plain: from inv = 1/nz to an ulp.
+// sx += nx/nz, sy += ny/nz; plain: from inv = 1/nz to an ulp, whose step is
+// right but for an nz of all ones, which no rounded reciprocal of a root is
+// (between 1 and 1 + 2^-52 there is no double); a Tilted's inv is right there.
 template <bool kPlain>
 BT_DEV void add_slope(double& sx, double& sy, double nx, double ny, double nz, double inv)
 {
@@ -1671,7 +1693,7 @@ BT_DEV void split_reflect(const Incidence& c, double& vx, double& vy, double& vz
 {
     const double ax = 2*c.alpha*c.nx, ay = 2*c.alpha*c.ny, az = 2*c.alpha*c.nz;
     if constexpr (kPlain) {
-        const double inv = recip_refine(c.n1, c.root);
+        const double inv = recip_refine(c.n1, c.root);   // as in add_slope
         vx = vx - div_plain_signed(ax, c.n1, inv);
         vy = vy - div_plain_signed(ay, c.n1, inv);
         vz = vz - div_plain_signed(az, c.n1, inv);

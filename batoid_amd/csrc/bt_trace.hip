@@ -263,6 +263,21 @@ __global__ __launch_bounds__(kBlock) void k_check_sqrt(
     out[n + i] = cr_rsqrt(x[i]);
 }
 
+// num/sqrt(x) as the normals of conics and spheres take x/r and y/r, and
+// num/x from a reciprocal that is about 2^-46 off, as the conics' r/(R sqrt(u)).
+__global__ __launch_bounds__(kBlock) void k_check_quotients(
+    const double* __restrict__ num, const double* __restrict__ x, double* __restrict__ out,
+    int64_t n)
+{
+    const int64_t i = ray_index();
+    if (i >= n) return;
+    double h;
+    const double root = sqrt_plain(x[i], h);
+    out[i] = div_plain_signed(num[i], root, recip_root(root, h));
+    const double off = recip_plain(x[i]) * (1.0 + ((i & 1) ? 0x1p-46 : -0x1p-46));
+    out[n + i] = div_plain_signed(num[i], x[i], recip_nearest(x[i], off));
+}
+
 // ---------------------------------------------------------------------------
 // Host helpers
 // ---------------------------------------------------------------------------
@@ -600,6 +615,16 @@ int bt_check_sqrt(const double* x, double* out, int64_t n, void* stream)
     hipLaunchKernelGGL(k_check_sqrt, dim3(grid_for(n)), dim3(kBlock), 0, as_stream(stream),
                        x, out, n);
     return check_launch("bt_check_sqrt");
+}
+
+int bt_check_quotients(const double* num, const double* x, double* out, int64_t n, void* stream)
+{
+    if (n > 0 && (!num || !x || !out)) return fail(BT_E_NULL, "bt_check_quotients: null argument");
+    if (n < 0) return fail(BT_E_SIZE, "bt_check_quotients: negative n");
+    if (n == 0) return 0;
+    hipLaunchKernelGGL(k_check_quotients, dim3(grid_for(n)), dim3(kBlock), 0, as_stream(stream),
+                       num, x, out, n);
+    return check_launch("bt_check_quotients");
 }
 
 }  // extern "C"

@@ -530,6 +530,11 @@ int bt_obsc_contains(const bt_obsc* obsc, int obsc_len, const double* x,
  * exists to test that and has no counterpart in the reference.            */
 int bt_check_sqrt(const double* x, double* out, int64_t n, void* stream);
 
+/* Likewise the quotients of the plain form (bt_device.h), for x and num away
+ * from the ends of the exponent range: out[0:n] = num/sqrt(x) and out[n:2n] =
+ * num/x, each from a reciprocal refined as the surface normals refine theirs. */
+int bt_check_quotients(const double* num, const double* x, double* out, int64_t n, void* stream);
+
 /* ---- RayVector field operations -----------------------------------------
  * Replace CPPRayVector.positionAtTime / propagateInPlace / phase /
  * amplitude / sumAmplitude (src/rayVector.cpp:26-222,
