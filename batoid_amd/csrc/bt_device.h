@@ -462,10 +462,11 @@ BT_DEV void table_point(SurfPtr s, double x, double y, double& sag, double& nx,
         }
         const double dx = s->p[2], dy = s->p[3], rx = s->p[4], ry = s->p[5];
         const double x0 = s->p[0], y0 = s->p[1];
-        // not the correctly rounded 1/dx and 1/dy (0: not given)
+        // not 1/dx and 1/dy to less than 2^-53, which the correctly rounded ones
+        // are and the quotients need (0: not given)
         if (!plain_exponent(dx) || !plain_exponent(dy)
-            || !(fabs(__builtin_fma(-dx, rx, 1.0)) <= 0x1p-53)
-            || !(fabs(__builtin_fma(-dy, ry, 1.0)) <= 0x1p-53))
+            || !(fabs(__builtin_fma(-dx, rx, 1.0)) < 0x1p-53)
+            || !(fabs(__builtin_fma(-dy, ry, 1.0)) < 0x1p-53))
             rg.leave();
         const double ux = x - x0, uy = y - y0;
         const double fx = floor(div_plain(ux, dx, rx)), fy = floor(div_plain(uy, dy, ry));
