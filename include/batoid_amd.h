@@ -72,7 +72,8 @@ typedef struct bt_rays {
  *   BICUBIC      p = {x0, y0, dx, dy, 1/dx, 1/dy}; n1 = nx, n2 = ny;
  *                flags = use_nan; the reciprocals are optional (0 where not
  *                given; one that is not 1/dx to less than 2^-53, as the
- *                correctly rounded one is, is not used) and change no result;
+ *                correctly rounded one is, is not used) and change no result,
+ *                but each point of the table takes two divisions without;
  *                a0..a3 = z, dzdx, dzdy, d2zdxdy row-major [ny][nx]
  *                                                         table.cpp:58-158
  *   POLYNOMIAL   p = {xorigin, yorigin}; n1 = xsize, n2 = ysize;
