@@ -824,10 +824,11 @@ __global__ __launch_bounds__(64, 1) void k_psf_gemm_batch(
     }
 }
 
-// amp[s][j][i] = sum over the segment's items of partial[item][i][j], FP64.
-// One lane per pixel where segments and pixels fill the chip by themselves
-// (a segment's few items in item order, four reads in flight), else the
-// lanes of reduce_splits.
+// amp[s][j][i] = sum over the segment's items of partial[item][i][j], FP64,
+// in the order of reduce_splits<8>: eight sums of every eighth item, then
+// those.  One lane per pixel keeps all eight (L = 1) where segments and pixels
+// fill the chip by themselves, else eight lanes take one each: the same sums,
+// so a segment's image does not depend on what else is in the call.
 template <int L>
 __global__ __launch_bounds__(kBlock) void k_psf_reduce_batch(
     const float* __restrict__ partial, const SegRange* __restrict__ ranges, int nseg, int nx,
@@ -848,15 +849,21 @@ __global__ __launch_bounds__(kBlock) void k_psf_reduce_batch(
     if constexpr (L > 1) {
         reduce_splits<L>(p, stride, r.first, last, live, out);
     } else if (live) {
-        double re = 0.0, im = 0.0;
-#pragma unroll 4
-        for (int k = r.first; k < last; k++) {
-            const float2 v = p[k * stride];
-            re += (double)v.x;
-            im += (double)v.y;
+        double re[8] = {}, im[8] = {};
+        for (int k = r.first; k < last; k += 8) {
+#pragma unroll
+            for (int g = 0; g < 8; g++) {
+                if (k + g >= last) break;
+                const float2 v = p[(k + g) * stride];
+                re[g] += (double)v.x;
+                im[g] += (double)v.y;
+            }
         }
-        out[0] = re;
-        out[1] = im;
+        double sre = 0.0, sim = 0.0;
+#pragma unroll
+        for (int g = 0; g < 8; g++) { sre += re[g]; sim += im[g]; }
+        out[0] = sre;
+        out[1] = sim;
     }
 }
 

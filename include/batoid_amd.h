@@ -657,7 +657,8 @@ int bt_huygens_gemm_noalloc(bt_rays rays, const double* p0, const double* a1,
  * allocation, no memset.  Rays are summed in work items of `chunk` rays (a
  * multiple of 8) that two waves for each of `nwg` (0: 512) take from a queue;
  * a result does not depend on who takes an item, and the items of one segment
- * are added in FP64 in a fixed order.
+ * are added in FP64 in an order of their own: every eighth one, in item order,
+ * then these eight sums.  A segment's image does not depend on the others.
  * `amp_out` receives [nseg][ny][nx][2] complex128.                         */
 typedef struct bt_psf_segment {
     int64_t begin, end;
