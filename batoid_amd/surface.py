@@ -266,15 +266,24 @@ def _horner_trim(tables):
     depend on it."""
     out = []
     for flat, nx, ny in tables:
-        flat = np.ascontiguousarray(flat, dtype=np.float64).ravel()
-        if ny > 0 and nx > 0:
-            rows = flat[:nx * ny].reshape(ny, nx).view(np.uint64) != 0
-            lens = [int(np.flatnonzero(row)[-1]) + 1 if row.any() else 0 for row in rows]
-        else:
-            lens = [0] * max(ny, 0)
-        last = max([i for i, n in enumerate(lens) if n > 0], default=-1)
-        out += [last] + lens
+        lens = []
+        for row in _rows(flat, nx, ny).view(np.uint64).tolist():
+            n = nx
+            while n and not row[n - 1]:
+                n -= 1
+            lens.append(n)
+        last = len(lens) - 1
+        while last >= 0 and not lens[last]:
+            last -= 1
+        out.append(last)
+        out += lens
     return np.array(out, dtype=np.int32)
+
+
+def _rows(flat, nx, ny):
+    """The ny x nx table that ``flat`` starts with."""
+    nx, ny = max(nx, 0), max(ny, 0)
+    return np.ascontiguousarray(flat, dtype=np.float64).ravel()[:nx * ny].reshape(ny, nx)
 
 
 def _horner_streams(tables, trim):
@@ -282,25 +291,24 @@ def _horner_streams(tables, trim):
     (include/batoid_amd.h, POLYNOMIAL): ``trim`` itself and what follows it in
     a3, as one int32 array.  A table of no coefficients or of more than 64
     quads (a full 16 x 16 table) has no stream."""
-    heads = np.zeros(3, dtype=[("nquad", "<i4"), ("first", "<i4"), ("row_ends", "<u8")])
-    data, k = [], 0
-    for head, (flat, nx, ny) in zip(heads, tables):
-        last, lens = int(trim[k]), trim[k + 1:k + 1 + ny]
-        k += 1 + ny
-        flat = np.ascontiguousarray(flat, dtype=np.float64).ravel()
-        quads = [max(-(-int(lens[i]) // 4), 1) for i in range(last, -1, -1)]
+    head, data, k = [0] * 16, [], 0      # three bt_poly_stream in 64 bytes
+    lens = trim.tolist()
+    for which, (flat, nx, ny) in enumerate(tables):
+        live = lens[k] + 1
+        quads = [max((n + 3) >> 2, 1) for n in lens[k + live:k:-1]]
+        k += 1 + max(ny, 0)
         if not 0 < sum(quads) <= 64:
             continue
-        head["nquad"] = sum(quads)
-        head["first"] = len(data)
-        head["row_ends"] = sum(1 << int(q - 1) for q in np.cumsum(quads))
-        for i, q in zip(range(last, -1, -1), quads):
-            row = flat[i * nx:i * nx + int(lens[i])][::-1]
-            data += [0.0] * (4 * q - len(row)) + row.tolist()
+        nquad, first, row_ends = 0, len(data), 0
+        for row, q in zip(_rows(flat, nx, live)[::-1].tolist(), quads):
+            row += [0.0] * (4 * q - nx)
+            data += row[4 * q - 1::-1]
+            nquad += q
+            row_ends |= 1 << (nquad - 1)
+        head[4 * which:4 * which + 4] = nquad, first, row_ends & 0xffffffff, row_ends >> 32
     data += [0.0] * 4
-    pad = np.zeros(-len(trim) % 16, dtype=np.int32)
-    return np.concatenate([trim, pad, heads.view(np.int32), np.zeros(4, dtype=np.int32),
-                           np.array(data, dtype=np.float64).view(np.int32)])
+    head = np.array([0] * (-len(lens) % 16) + head, dtype=np.uint32).view(np.int32)
+    return np.concatenate([trim, head, np.array(data).view(np.int32)])
 
 
 class Zernike(Surface):
