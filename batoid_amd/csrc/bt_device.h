@@ -69,8 +69,8 @@ using TablePtr = const BT_GLOBAL double*;
 // true) runs these alone and notes in a Range what could have left their
 // range; a wave votes once on its lanes' Ranges, and only if one left it is
 // the work done again, by the whole wave, in the full form, whose roots and
-// divisions are the compiler's sequences.  The full form (the on-axis ray
-// r = 0, overflow) stays out of the plain form's registers.
+// divisions are the compiler's sequences.  The full form (overflow, rays that
+// leave an asphere's domain) stays out of the plain form's registers.
 //
 // A Range is two running extremes in vector registers, an instruction or two
 // per value noted: the compares and scalar masks of a test at each root cost
@@ -80,9 +80,8 @@ using TablePtr = const BT_GLOBAL double*;
 //    overflow, a NaN) and denominators;
 //  * the exponents of a ray's x and y at each surface and of its final
 //    velocity: nothing nonzero below 2^-383.  So x*x + y*y, whose root is
-//    taken without a note of its own, is 0 (a NaN slope follows, which is
-//    noted) or at least 2^-766, and no remainder n - d q of a quotient
-//    underflows.  (A difference of two doubles is 0 or at least an ulp of
+//    taken without a note of its own, is 0 (see off_axis) or at least 2^-766,
+//    and no remainder n - d q of a quotient underflows.  (A difference of two doubles is 0 or at least an ulp of
 //    theirs, so tiny values come only from tiny values; where a Newton
 //    iterate alone is tiny, its slopes are lost beside the other terms.)
 // ---------------------------------------------------------------------------
@@ -559,6 +558,16 @@ BT_DEV double even_terms(CoefPtr c, int n, double result, double term, double r2
     return result;
 }
 
+// x*x + y*y for the plain form's root.  A ray at the vertex (0) goes on with
+// 2^-767, whose slopes are lost beside 1: the normal is (+-0, +-0, 1), and
+// arrival_normal gives the zeros their sign, which nothing before depends on.
+// The chief ray of every centred field meets the vertices; while its wave ran
+// the full form after the plain one, 49 rays through twelve interfaces took 68
+// us, 38 in the full form alone, 34 now (with three perturbed mirrors 181, 122,
+// 81).  Others pay 1 % (a NaN is taken for 2^-767, too, but no ray gets here
+// with one before a root of its discriminant or sag was noted).
+BT_DEV double off_axis(double r2) { return __builtin_fmax(r2, 0x1p-767); }
+
 // Sag and / or normal of a Quadric (kAsphere false) or an Asphere (true) at
 // one point: quadric.cpp:18-39, asphere.cpp:37-62.  `inv`: 1/nz to an ulp,
 // or 0.  Bound by FP64 issue: the normal's three divisions start from the
@@ -581,14 +590,14 @@ BT_DEV void conic_point(SurfPtr s, double x, double y, double& sag, double& nx,
         }
         if constexpr (kNormal) {
             double hr, hu;
-            const double r = sqrt_plain(r2, hr);
+            const double r = sqrt_plain(off_axis(r2), hr);
             const double u = 1-r*r*cp1R2;
             const double d = R*sqrt_plain(u, hu);
             const double y0 = (hu + hu) * (R*s->p[3]);   // 1/sqrt(u) * (R * 1/R/R)
             double dzdr = div_plain(r, d, recip_nearest(d, y0));
             if constexpr (kAsphere) dzdr = even_terms((CoefPtr)s->a1, s->n1, dzdr, r, r*r);
             const double w = 1+dzdr*dzdr;
-            rg.above(w);                                 // a NaN for r2 = 0 or u = 0
+            rg.above(w);                                 // a NaN for u = 0
             nz = rsqrt_plain(w, inv);
             const double yr = recip_root(r, hr);
             nx = -div_plain_signed(x, r, yr)*dzdr*nz;
@@ -625,14 +634,14 @@ BT_DEV void sphere_normal(SurfPtr s, double x, double y, double& nx, double& ny,
     const double rsqr = x*x + y*y;
     if constexpr (kPlain) {
         double hr, hu;
-        const double r = sqrt_plain(rsqr, hr);
+        const double r = sqrt_plain(off_axis(rsqr), hr);
         const double rat = r*Rinv;
         const double u = 1-rat*rat;
         const double su = sqrt_plain(u, hu);
         const double dzdr = div_plain(rat, su, recip_root(su, hu));
         const double w = 1+dzdr*dzdr;
         if (!plain_exponent(Rinv)) rg.leave();
-        rg.above(w);                                     // a NaN for rsqr = 0 or u = 0
+        rg.above(w);                                     // a NaN for u = 0
         nz = rsqrt_plain(w, inv);
         const double yr = recip_root(r, hr);
         nx = -div_plain_signed(x, r, yr)*dzdr*nz;
@@ -1808,6 +1817,16 @@ BT_DEV void arrival_normal(SurfPtr surf, const Arrival& a, double& nx, double& n
         double sag;
         if constexpr (!kPlain) surf = anew(surf);    // after Newton only in the full form
         surf_point<K, kPlain, false, true>(surf, a.x, a.y, sag, nx, ny, nz, rg);
+    }
+    if constexpr (kPlain) {                          // quadric.cpp:29, asphere.cpp:50
+        const bool vertex = (a.x == 0.0) & (a.y == 0.0);
+        if (__builtin_expect(__any(vertex), 0)) {
+            const int kind = surf->kind;
+            if (kind == BT_SPHERE || kind == BT_QUADRIC || kind == BT_ASPHERE) {
+                nx = vertex ? 0.0 : nx;
+                ny = vertex ? 0.0 : ny;
+            }
+        }
     }
 }
 

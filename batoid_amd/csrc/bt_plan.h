@@ -130,7 +130,7 @@ __device__ __forceinline__ void trace_steps(bt_plan plan, bt_rays in, int64_t i,
 
 // Kernels whose waves run the plan in the plain form, vote once at its end,
 // and read their rays again for the full form if a lane left the plain range
-// (a chief ray with x = y = 0 exactly, an overflow): the full form shares no
+// (an overflow, a ray beyond an asphere's domain): the full form shares no
 // live register with the plain loop.  (A vote at each step kept the ray twice
 // and cost a wave of occupancy: 1.96 against 1.78 ms for 1e7 rays of the
 // analytic kernel.)  Kernel times before and after, at the same clocks:
