@@ -104,12 +104,10 @@ struct Range {
         low = min(min(low, __builtin_amdgcn_frexp_exp(a)), __builtin_amdgcn_frexp_exp(b));
     }
     __device__ __forceinline__ void leave() { high = ~0u; }
-    // roots' arguments from 2^-767 to 2^857, slopes' below 2^601, and nothing
-    // nonzero below 2^-383
-    __device__ __forceinline__ bool plain() const
-    {
-        return (high < ((1023u + 601u) << 20)) & (low >= -382);
-    }
+    // roots' arguments from 2^-767 to 2^857, slopes' below 2^601
+    __device__ __forceinline__ bool left() const { return high >= ((1023u + 601u) << 20); }
+    // that, and nothing nonzero below 2^-383
+    __device__ __forceinline__ bool plain() const { return !left() & (low >= -382); }
 };
 
 

@@ -125,6 +125,8 @@ __device__ __forceinline__ void trace_steps(bt_plan plan, bt_rays in, int64_t i,
         const int olen = st->obsc_len;
         if (olen > 0 && !r.vig)
             r.vig = obsc_contains(obscs + st->obsc, olen, r.x, r.y);
+        if constexpr (kPlain && K == kKindsAnalytic)
+            if (__any(rg.left())) break;        // the full form decides
     }
 }
 
@@ -133,7 +135,12 @@ __device__ __forceinline__ void trace_steps(bt_plan plan, bt_rays in, int64_t i,
 // (an overflow, a ray beyond an asphere's domain): the full form shares no
 // live register with the plain loop.  (A vote at each step kept the ray twice
 // and cost a wave of occupancy: 1.96 against 1.78 ms for 1e7 rays of the
-// analytic kernel.)  Kernel times before and after, at the same clocks:
+// analytic kernel.)  A wave of the analytic kernel stops at the step where a root
+// left the range: a 512 x 512 beam 1.6 times as wide as the pupil of a
+// 20-interface corrector, 29 % of which fails, takes 152 to 172 us, 203 to 208
+// with the whole plan in both forms, 138 in the full form alone; others pay
+// 0.4 % (2 % for the Sums, whose failing rays mostly leave the Bicubic's grid,
+// which is no cause for the full form).  Kernel times before and after, at the same clocks:
 // 2.01 -> 1.78 ms (analytic, 1e7 rays x 12), 0.86 -> 0.70 ms (three perturbed
 // mirrors, 1e6), 1.18 -> 1.08 (the same, conic start, 3e6), 0.49 -> 0.46
 // (freeform, 3e5), 41 -> 35 us (162 rays).  Bound by FP64 issue.  The
