@@ -125,7 +125,7 @@ MED_CONST, MED_TABLE, MED_SELLMEIER, MED_SUMITA, MED_AIR = range(5)
  OB_UNION, OB_INTERSECTION) = range(8)
 ACT_INTERSECT, ACT_REFLECT, ACT_REFRACT = range(3)
 ACT_SPLIT = 3
-CHAIN_FILTERED, CHAIN_NO_OUTPUT = 1, 2
+CHAIN_FILTERED, CHAIN_NO_OUTPUT, CHAIN_KEEP = 1, 2, 4
 START_REFERENCE, START_CONIC, START_MLP = range(3)
 PLAN_NO_REFRACT = 1
 PLAN_FAST_START = 2

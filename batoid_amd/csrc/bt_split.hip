@@ -246,10 +246,12 @@ void k_split_chains(ChainPtr chains, double min_flux, int niter)
         chain_ray<K, false>(steps, nstep, rays, i, min_flux, first_live, niter, c, rg);
     }
     if (flags & BT_CHAIN_NO_OUTPUT) return;
+    const bool keep = (flags & BT_CHAIN_KEEP) != 0;
+    if (keep && (rays.vignetted[i] != 0 || !(rays.flux[i] >= min_flux))) return;
     rays.flux[i] = c.flux;
     rays.vignetted[i] = c.r.vig;
     rays.failed[i] = c.r.fail;
-    if (first_live && c.drop) return;           // no later pass reads the rest
+    if (first_live && c.drop && !keep) return;  // no later pass reads the rest
     rays.x[i] = c.r.x; rays.y[i] = c.r.y; rays.z[i] = c.r.z;
     rays.vx[i] = c.r.vx; rays.vy[i] = c.r.vy; rays.vz[i] = c.r.vz;
     rays.t[i] = c.r.t;

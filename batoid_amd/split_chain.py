@@ -25,12 +25,14 @@ from .rayVector import RayVector
 
 class _Set:
     """A ray set: the steps of its chain as (interface, reversed, reflected
-    set or None), and where it started."""
-    __slots__ = ("steps", "rays", "start", "leaves", "first")
+    set or None), where it started (None: the caller's own set), and whether
+    the filter applies to it before its first step."""
+    __slots__ = ("steps", "rays", "start", "leaves", "first", "filtered")
 
     def __init__(self, start):
         self.steps, self.start = [], start
         self.rays, self.leaves, self.first = None, False, 0
+        self.filtered = start is not None
 
 
 class _Token:
@@ -91,6 +93,8 @@ def _walk(optic, inputs, minFlux, sets):
             item = optic.items[index]
             if item.skip:
                 results = [([], [w[2]]) if w[3] else ([w[2]], []) for w in entries]
+                for w in entries:            # the filter follows a skipped item too
+                    w[2].set.filtered |= not w[2].set.steps
             elif hasattr(item, 'items'):
                 results = _walk(item, [(w[2], w[3]) for w in entries], minFlux, sets)
             else:
@@ -211,8 +215,11 @@ def trace_split(optic, rv, reverse, minFlux, bound):
                 part = group[at:at + 65535]
                 groups.append((len(chains), len(part), k))
                 for s in part:
-                    flags = (0 if s is root else _lib.CHAIN_FILTERED) | (
-                        0 if s.leaves or s is root else _lib.CHAIN_NO_OUTPUT)
+                    flags = _lib.CHAIN_FILTERED if s.filtered else 0
+                    if s is root:
+                        flags |= _lib.CHAIN_KEEP if s.filtered else 0
+                    elif not s.leaves:
+                        flags |= _lib.CHAIN_NO_OUTPUT
                     chains.append(_lib.BtChain(
                         steps.data_ptr() + s.first * ctypes.sizeof(_lib.BtChainStep),
                         len(s.steps), flags, s.rays._rays))

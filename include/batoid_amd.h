@@ -380,6 +380,9 @@ typedef struct bt_chain_step {
 /* A ray set and the steps it takes (DEVICE array `steps`).                 */
 #define BT_CHAIN_FILTERED  1    /* the filter already applies to `rays`     */
 #define BT_CHAIN_NO_OUTPUT 2    /* the continuing rays are not written back */
+#define BT_CHAIN_KEEP      4    /* with FILTERED: rays dropped before the first
+                                   step stay as they are, those that a step
+                                   drops are written back in full           */
 typedef struct bt_chain {
     const bt_chain_step* steps;
     int32_t nstep;
@@ -492,7 +495,8 @@ int bt_select_scatter_many(const bt_rays* in, const bt_rays* out, int nset, int6
  * further: its later reflected parts are marked vignetted and nothing else
  * of them is written; a reflected part that the filter drops is written as
  * its flux and flags.  The continuing rays are written back in place, of a
- * dropped ray of a filtered set the flux and flags only.  `kinds`:
+ * dropped ray of a filtered set (without BT_CHAIN_KEEP) the flux and flags
+ * only.  `kinds`:
  * BT_PLAN_ANALYTIC or BT_PLAN_FLAT_SUMS where every step's surface allows,
  * as for a plan.                                                           */
 int bt_split_chains(const bt_chain* chains, int nchain, int64_t n, double min_flux, int niter,
