@@ -187,16 +187,20 @@ class PSFBatch:
 
     def autotune(self, chunks=(1024, 2048, 4096, 8192), nwgs=(256, 512, 768, 1024), reps=3):
         """Pick the (chunk, workgroups) pair with the shortest eager run on
-        this batch; returns {(chunk, nwg): ms}.  Results do not depend on the
-        choice beyond FP32 summation order within a segment."""
+        this batch, the smallest chunk among those within 2 % of it; returns
+        {(chunk, nwg): ms}.  Results do not depend on the choice beyond FP32
+        summation order within a segment, whose error grows with the chunk
+        (384 segments of 1e4 to 2e5 rays: 9.3e-7 relative L2 with chunks of
+        1024 rays, 1.2e-6 with 2048, which took 0.7 % less)."""
         graph = self.graph is not None
         timings = {}
         for c in chunks:
             for w in nwgs:
                 self._configure(c, w)
                 timings[(c, w)] = self.time(reps)
-        best = min(timings, key=timings.get)
-        self._configure(*best)
+        limit = 1.02 * min(timings.values())
+        self._configure(*min((k for k, ms in timings.items() if ms <= limit),
+                             key=lambda k: (k[0], timings[k])))
         if graph:
             self.capture()
         return timings

@@ -762,7 +762,7 @@ def bench_batch(reps=5, nets=None):
     torch.cuda.synchronize()
     log(f"batch: {nseg} segments, {b.n} rays, set up in {time.perf_counter() - t0:.1f} s")
     timings = b.autotune(reps=2)
-    best = min(timings, key=timings.get)
+    best = (b.chunk, b.nwg)
     log(f"batch autotune: best chunk {best[0]}, {best[1]} workgroups, {timings[best]:.2f} ms")
     eager_ms = b.time(reps)
     b.capture()
