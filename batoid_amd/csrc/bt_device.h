@@ -1750,7 +1750,7 @@ struct Arrival {
 // A rotation by nothing: the unit matrix, zeros of either sign (tested on the
 // scalar unit).  Its products are exact, so 12 FMAs give the bits of the 18
 // products and 12 sums, signed zeros and NaNs included.  Only in the kernels
-// of analytic surfaces, which issue bounds: 1786 -> 1753 us for 1e7 rays
+// of analytic surfaces, which issue bounds: 1780 -> 1745 us for 1e7 rays
 // through twelve Interfaces; the freeform kernel was 2 % slower with it.
 template <class Frame>
 BT_DEV bool unrotated(Frame m)

@@ -8,15 +8,6 @@
 
 namespace bt {
 
-// Every step of a plan applied while the ray stays in registers.  A ray's
-// wavelength never changes, so the index of the plan's (first) dispersive
-// medium is evaluated once per ray up front.
-//
-// Mode 0: reference starts only.  Mode 1: CONIC starts honoured (an MLP step
-// runs as CONIC).  Mode 2: MLP starts too; MLP inference is a wave-wide MFMA
-// product, so in this variant every lane of a wave stays in the step loop
-// (lanes past the end work on a copy of the last ray and store nothing).
-//
 // The network's input at an MLP step: the ray's point on the surface's base
 // conic and its direction, in the step's local frame (the frame change is
 // apply_interaction's).
@@ -55,9 +46,6 @@ __device__ __forceinline__ void mlp_features(StepPtr st, SurfPtr surf, const Ray
 // compiler would settle for two).  Mode 0 at three, four and five waves: 621,
 // 573, 655 us (1e6 rays, three perturbed mirrors), 320, 304, 372 (3e5,
 // freeform); the conic start on the first, 3e6 rays: 1002, 918, 1305.
-// Networks a plan kernel keeps in LDS (45 KB per workgroup).
-constexpr int kMlpLds = 4;
-
 template <int Mode, int K>
 constexpr int plan_waves_per_simd()
 {
@@ -66,8 +54,18 @@ constexpr int plan_waves_per_simd()
     return Mode == 0 ? 4 : 3;     // kKindsAll, kKindsFlatSums
 }
 
-// Ray i of `in` through every step of the plan, in the plain form (what may
-// have left its range noted in `rg`) or the full one.
+// Networks a plan kernel keeps in LDS (45 KB per workgroup).
+constexpr int kMlpLds = 4;
+
+// Ray i of `in` through every step of the plan while it stays in registers, in
+// the plain form (what may have left its range noted in `rg`) or the full one.
+// A ray's wavelength never changes, so the index of the plan's (first)
+// dispersive medium is evaluated once per ray up front.
+//
+// Mode 0: reference starts only.  Mode 1: CONIC starts honoured (an MLP step
+// runs as CONIC).  Mode 2: MLP starts too; MLP inference is a wave-wide MFMA
+// product, so in this variant every lane of a wave stays in the step loop
+// (lanes past the end work on a copy of the last ray and store nothing).
 template <int Mode, int K, bool kPlain>
 __device__ __forceinline__ void trace_steps(bt_plan plan, bt_rays in, int64_t i,
                                             int niter, int need_w, const MlpPacked* nets,

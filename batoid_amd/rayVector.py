@@ -143,15 +143,6 @@ class RayVector:
         optic.py:1256-1266)."""
         return _SelectCounts(rvs, minFlux)
 
-    @staticmethod
-    def _select_many(rvs, minFlux):
-        """``[rv._select(minFlux) for rv in rvs]`` with one host
-        synchronisation for all the counts instead of one per RayVector."""
-        if not rvs:
-            return []
-        sel = _SelectCounts(rvs, minFlux)
-        return [sel.scatter(i, m) for i, m in enumerate(sel.counts.tolist())]
-
     @classmethod
     def fromTorch(cls, x, y, z, vx, vy, vz, t, wavelength, flux, vignetted, failed,
                   coordSys=globalCoordSys):

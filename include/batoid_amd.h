@@ -103,7 +103,9 @@ enum bt_surface_kind {
 #define BT_POLY_STREAMS 1
 
 typedef struct bt_poly_stream {
-    int32_t nquad;            /* quads of coefficients; 0: table without stream */
+    int32_t nquad;            /* quads of coefficients; 0: table without stream
+                                 (for readers of a record; kernels go by
+                                 row_ends)                                     */
     int32_t first;            /* its first coefficient's index in the streams */
     uint64_t row_ends;        /* bit k: quad k ends a row, the last too
                                  (nquad <= 64); 0: table without stream */
