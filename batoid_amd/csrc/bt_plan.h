@@ -40,8 +40,8 @@ __device__ __forceinline__ void mlp_features(StepPtr st, SurfPtr surf, const Ray
 }
 
 // Waves per SIMD: the analytic-kinds kernels of modes 0 and 1 are held to
-// six (79 and 80 VGPRs), the Sum(Asphere, Polynomial, Bicubic) kernels to
-// four (128 VGPRs; mode 0 spills 18 words outside its Newton loops), the
+// six (77 and 79 VGPRs), the Sum(Asphere, Polynomial, Bicubic) kernels to
+// four (128 VGPRs; mode 0 spills 16 words outside its Newton loops), the
 // others of mode 0 to four and of modes 1 and 2 to three (left alone the
 // compiler would settle for two).  Mode 0 at three, four and five waves: 621,
 // 573, 655 us (1e6 rays, three perturbed mirrors), 320, 304, 372 (3e5,
@@ -139,7 +139,8 @@ __device__ __forceinline__ void trace_steps(bt_plan plan, bt_rays in, int64_t i,
 // with the whole plan in both forms, 138 in the full form alone; others pay
 // 0.4 % (2 % for the Sums, whose failing rays mostly leave the Bicubic's grid,
 // which is no cause for the full form).  Kernel times before and after, at the same clocks:
-// 2.01 -> 1.78 ms (analytic, 1e7 rays x 12), 0.86 -> 0.70 ms (three perturbed
+// 2.01 -> 1.78 ms (analytic, 1e7 rays x 12; 1.84 with quotients right for every
+// denominator and vertices in the plain form), 0.86 -> 0.70 ms (three perturbed
 // mirrors, 1e6), 1.18 -> 1.08 (the same, conic start, 3e6), 0.49 -> 0.46
 // (freeform, 3e5), 41 -> 35 us (162 rays).  Bound by FP64 issue.  The
 // nested-Sum and learned-start kernels hold the full form alone: theirs is as

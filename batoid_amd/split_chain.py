@@ -12,9 +12,9 @@ pass (bt_split_chains), its reflected parts going to their own buffers.
 
 For 998,388 rays through the twelve-interface telescope with 2 % reflective
 glass (44 paths out) three launches take the place of 279 of one Interface
-each, 36 us apiece (132 B a ray and Interface of traffic): a call takes 7.4
-instead of 12.0 ms, of which the chains are 4.6 (FP64 issue), the copies out
-0.9; for 10,368 rays, where the launches' host side was the time, 2.2 instead
+each, 36 us apiece (132 B a ray and Interface of traffic): a call takes 7.3
+instead of 12.0 ms, of which the chains are 4.7 (FP64 issue), the copies out
+0.8; for 10,368 rays, where the launches' host side was the time, 2.2 instead
 of 6.1 ms."""
 import ctypes
 

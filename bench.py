@@ -38,11 +38,11 @@ MEASURED_TRAFFIC_PER_RAY = 124.05
 # FP64 flops per ray of the same kernel on this workload: 64 lanes x
 # (ADD + MUL + 2 FMA) FP64 wave instructions (SQ_INSTS_VALU_*_F64), same file
 # (current build's figure; issued lanes, an upper bound on useful flops).
-FP64_FLOP_PER_RAY = 5650.5
+FP64_FLOP_PER_RAY = 5740.5
 # The same two figures for the C3 kernel (perturbed TMA, reference start),
 # from profiles/trace_plan_c3_perturbed_tma_1e7.md.
-C3_FP64_FLOP_PER_RAY = 15303.0
-C3_TRAFFIC_PER_RAY = 238.3
+C3_FP64_FLOP_PER_RAY = 15450.6
+C3_TRAFFIC_PER_RAY = 214.5
 # Ray generation writes 9 FP64 columns and 2 flag bytes per ray.
 RAYGEN_BYTES_PER_RAY = 9 * 8 + 2
 
