@@ -157,7 +157,8 @@ BT_DEV double recip_nearest(double d, double y0)
     return __builtin_fma(__builtin_fma(-d, y, 1.0), odd(y), y);
 }
 
-// 1/d to within an ulp.
+// 1/d to within an ulp.  With div_plain the steps are the compiler's division's,
+// and so are the results.
 BT_DEV double recip_plain(double d)
 {
     return recip_refine(d, recip_refine(d, __builtin_amdgcn_rcp(d)));
